@@ -8,10 +8,10 @@
 //                           (+ for Q4_K: sum_b (-dmin * m)(row, b) * xsum_delta[h, b])   (3417-3453)
 // with r_h = h * (qk_nope + v_head) the first kv_b row of head h, q rows of qk_nope + qk_rope, and
 // w(row, k) the canonical dequantized element.  These are small (DeepSeek-V2-Lite: 16 heads, kv_b
-// [4096, 512]) and latency-bound, so each output is one thread (or one wave for the v product) with
-// the sums in index order.
+// [4096, 512]) and latency-bound.
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
+#include "qlin_values8.hpp"
 
 namespace qlin {
 namespace {
@@ -27,69 +27,126 @@ __global__ __launch_bounds__(256) void embedding_kernel(const int *__restrict__ 
         o[k] = block_value<T>(row + static_cast<size_t>(k / BE) * BB, k % BE);
 }
 
+// The three absorptions are small (DeepSeek-V2-Lite: 16 heads, kv_b [4096, 512], 1.2 MB) and bound by
+// latency, so each spreads its rows over enough threads that every byte is requested in one or two
+// rounds.  With one thread per output and the rows in turn (128 dependent rounds of byte loads) q_nope
+// took 64 us and xsum_delta, one workgroup in all, 77 us; v, a wave per output with one element per
+// lane and round, 9.6 us.
+
+constexpr int kQCols = 64, kQThreads = 1024;
+
+// A workgroup per (head, 64 latent columns): thread (cg, ds) takes columns 8cg .. 8cg+7 of the head's
+// rows ds, ds + 128, ...; the rows' sums meet by lane shuffles, then in LDS in wave order.
 template <int T>
-__global__ __launch_bounds__(256) void absorb_q_nope_kernel(const float *__restrict__ q, const uint8_t *__restrict__ w,
-                                                            size_t rb, float *__restrict__ q_abs, int n_heads,
-                                                            int qk_nope, int qk_rope, int v_head, int kv_lora) {
-    constexpr int BE = Block<T>::elems, BB = Block<T>::bytes;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n_heads * kv_lora) return;
-    const int h = i / kv_lora, l = i - h * kv_lora;
-    const float *qh = q + static_cast<size_t>(h) * (qk_nope + qk_rope);
-    const uint8_t *col = w + static_cast<size_t>(h) * (qk_nope + v_head) * rb + static_cast<size_t>(l / BE) * BB;
-    float acc = 0.0f;
-    for (int d = 0; d < qk_nope; ++d) acc = fmaf(block_value<T>(col + static_cast<size_t>(d) * rb, l % BE), qh[d], acc);
-    q_abs[i] = acc;
-}
-
-// -dmin * m of 32-block b of a Q4_K row (the min term of every element of that block)
-__device__ __forceinline__ float q4k_min_coeff(const uint8_t *row, int b) {
-    const uint8_t *sb = row + static_cast<size_t>(b >> 3) * 144;
-    const uint32_t s0 = sb[4] | (sb[5] << 8) | (sb[6] << 16) | (static_cast<uint32_t>(sb[7]) << 24);
-    const uint32_t s1 = sb[8] | (sb[9] << 8) | (sb[10] << 16) | (static_cast<uint32_t>(sb[11]) << 24);
-    const uint32_t s2 = sb[12] | (sb[13] << 8) | (sb[14] << 16) | (static_cast<uint32_t>(sb[15]) << 24);
-    int sc, m;
-    q4k_scale_min(b & 7, s0, s1, s2, sc, m);
-    return -mul_rn(f16_bits_to_f32(ld_u16(sb + 2)), static_cast<float>(m));
-}
-
-__global__ __launch_bounds__(256) void absorb_xsum_delta_kernel(const float *__restrict__ q,
-                                                                const uint8_t *__restrict__ w, size_t rb,
-                                                                float *__restrict__ delta, int n_heads, int qk_nope,
-                                                                int qk_rope, int v_head, int nblk) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n_heads * nblk) return;
-    const int h = i / nblk, b = i - h * nblk;
+__global__ __launch_bounds__(kQThreads) void absorb_q_nope_kernel(const float *__restrict__ q,
+                                                                  const uint8_t *__restrict__ w, size_t rb,
+                                                                  float *__restrict__ q_abs, int qk_nope, int qk_rope,
+                                                                  int v_head, int kv_lora, int tiles) {
+    __shared__ float part[kQThreads / 64][kQCols];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int h = blockIdx.x / tiles, l0 = (blockIdx.x - h * tiles) * kQCols;
+    const int cg = tid & 7, ds = tid >> 3, k0 = l0 + 8 * cg;
     const float *qh = q + static_cast<size_t>(h) * (qk_nope + qk_rope);
     const uint8_t *rows = w + static_cast<size_t>(h) * (qk_nope + v_head) * rb;
-    float acc = 0.0f;
-    for (int d = 0; d < qk_nope; ++d) acc = fmaf(qh[d], q4k_min_coeff(rows + static_cast<size_t>(d) * rb, b), acc);
-    delta[i] = acc;
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
+    if (k0 < kv_lora) {
+        for (int d = ds; d < qk_nope; d += kQThreads / 8) {
+            Raw8<T> r;
+            raw8<T>(rows + static_cast<size_t>(d) * rb, k0, r);
+            const float qd = qh[d];
+            float v[8];
+            values8<T>(r, k0, v);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[i] = fmaf(v[i], qd, acc[i]);
+        }
+    }
+#pragma unroll
+    for (int off = 8; off < 64; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] += __shfl_xor(acc[i], off, 64);
+    if (lane < 8) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) part[wave][8 * cg + i] = acc[i];
+    }
+    __syncthreads();
+    if (tid < kQCols && l0 + tid < kv_lora) {
+        float v = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kQThreads / 64; ++u) v += part[u][tid];
+        q_abs[static_cast<size_t>(h) * kv_lora + l0 + tid] = v;
+    }
 }
 
+// -dmin * m of sub-block j from a Q4_K super-block's first 16 bytes (the min term of every element of
+// that 32-block)
+__device__ __forceinline__ float q4k_min_coeff(const u32x4 &hdr, int j) {
+    int sc, m;
+    q4k_scale_min(j, hdr.y, hdr.z, hdr.w, sc, m);
+    return -mul_rn(f16_bits_to_f32(hdr.x >> 16), static_cast<float>(m));
+}
+
+constexpr int kDThreads = 128;
+
+// A workgroup per (head, super-block): a thread per row, the super-block's 8 sums over the rows by
+// wave sums and LDS.
+__global__ __launch_bounds__(kDThreads) void absorb_xsum_delta_kernel(const float *__restrict__ q,
+                                                                      const uint8_t *__restrict__ w, size_t rb,
+                                                                      float *__restrict__ delta, int qk_nope,
+                                                                      int qk_rope, int v_head, int nsb) {
+    __shared__ float part[kDThreads / 64][8];
+    const int tid = threadIdx.x, h = blockIdx.x / nsb, s = blockIdx.x - h * nsb;
+    const float *qh = q + static_cast<size_t>(h) * (qk_nope + qk_rope);
+    const uint8_t *rows = w + static_cast<size_t>(h) * (qk_nope + v_head) * rb + static_cast<size_t>(s) * 144;
+    float acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+    for (int d = tid; d < qk_nope; d += kDThreads) {
+        const u32x4 hdr = ld16_a2(rows + static_cast<size_t>(d) * rb);
+        const float qd = qh[d];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] = fmaf(qd, q4k_min_coeff(hdr, j), acc[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = wave_sum(acc[j]);
+    if ((tid & 63) == 0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) part[tid >> 6][j] = acc[j];
+    }
+    __syncthreads();
+    if (tid < 8) delta[static_cast<size_t>(blockIdx.x) * 8 + tid] = part[0][tid] + part[1][tid];
+}
+
+// A wave per output row, 8 consecutive elements per lane: one round for kv_lora up to 512.
 template <int T>
 __global__ __launch_bounds__(256) void absorb_v_kernel(const uint8_t *__restrict__ w, size_t rb,
                                                        const float *__restrict__ latent,
                                                        const float *__restrict__ delta, float *__restrict__ attn,
                                                        int n_heads, int qk_nope, int v_head, int kv_lora) {
-    constexpr int BE = Block<T>::elems, BB = Block<T>::bytes;
     const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= n_heads * v_head) return;  // whole waves
     const int h = i / v_head, v = i - h * v_head;
     const uint8_t *row = w + (static_cast<size_t>(h) * (qk_nope + v_head) + qk_nope + v) * rb;
     const float *x = latent + static_cast<size_t>(h) * kv_lora;
     float acc = 0.0f;
-    for (int k = lane; k < kv_lora; k += 64)
-        acc = fmaf(block_value<T>(row + static_cast<size_t>(k / BE) * BB, k % BE), x[k], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) {
+    for (int k0 = 8 * lane; k0 < kv_lora; k0 += 512) {
+        Raw8<T> r;
+        raw8<T>(row, k0, r);
+        float xv[8], wv[8];
+        __builtin_memcpy(xv, x + k0, sizeof(xv));
+        values8<T>(r, k0, wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc = fmaf(wv[e], xv[e], acc);
         if constexpr (T == T_Q4_K) {
-            const int nblk = (kv_lora + 31) / 32;
-            const float *dh = delta + static_cast<size_t>(h) * nblk;
-            for (int b = 0; b < nblk; ++b) acc = fmaf(q4k_min_coeff(row, b), dh[b], acc);
+            if ((k0 & 31) == 0) {
+                const int b = k0 >> 5;
+                acc = fmaf(q4k_min_coeff(r.hdr, b & 7), delta[static_cast<size_t>(h) * (kv_lora / 32) + b], acc);
+            }
         }
-        attn[i] = acc;
     }
+    acc = wave_sum(acc);
+    if (lane == 0) attn[i] = acc;
 }
 
 template <template <int> class K, typename... Args>
@@ -112,8 +169,9 @@ template <int T> struct Embed {
 template <int T> struct QNope {
     static void run(const float *q, const uint8_t *w, size_t rb, float *q_abs, int nh, int qn, int qr, int vh, int kl,
                     hipStream_t s) {
-        hipLaunchKernelGGL(absorb_q_nope_kernel<T>, dim3((nh * kl + 255) / 256), dim3(256), 0, s, q, w, rb, q_abs,
-                           nh, qn, qr, vh, kl);
+        const int tiles = (kl + kQCols - 1) / kQCols;
+        hipLaunchKernelGGL(absorb_q_nope_kernel<T>, dim3(nh * tiles), dim3(kQThreads), 0, s, q, w, rb, q_abs, qn, qr,
+                           vh, kl, tiles);
     }
 };
 template <int T> struct AbsorbV {
@@ -143,10 +201,10 @@ hipError_t mla_absorb_q_nope(int type, const float *q, const uint8_t *w, size_t 
 
 hipError_t mla_absorb_q4_xsum_delta(const float *q, const uint8_t *w, size_t rb, float *delta, int n_heads,
                                     int qk_nope, int qk_rope, int v_head, int kv_lora, hipStream_t s) {
-    const int nblk = (kv_lora + 31) / 32;
-    if (n_heads == 0 || nblk == 0) return hipSuccess;
-    hipLaunchKernelGGL(absorb_xsum_delta_kernel, dim3((n_heads * nblk + 255) / 256), dim3(256), 0, s, q, w, rb,
-                       delta, n_heads, qk_nope, qk_rope, v_head, nblk);
+    const int nsb = kv_lora / 256;
+    if (n_heads == 0 || nsb == 0) return hipSuccess;
+    hipLaunchKernelGGL(absorb_xsum_delta_kernel, dim3(n_heads * nsb), dim3(kDThreads), 0, s, q, w, rb, delta, qk_nope,
+                       qk_rope, v_head, nsb);
     return hipGetLastError();
 }
 

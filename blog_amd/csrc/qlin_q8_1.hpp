@@ -61,6 +61,50 @@ __device__ __forceinline__ void quantize_block_q8_1(const float *src, int valid,
     quantize_block_q8_1(src, valid, out, out + 1, raw);
 }
 
+// One Q8_1 block by 8 consecutive lanes (all active): lane j = 0..7 takes the 4 values at index k0 of the
+// row src (those at in_dim or past it are 0) and writes their q; lane 0 writes (d, s).  The same bytes as
+// quantize_block_q8_1: the maximum and the integer sum have no order, and the raw sum's adds pair the
+// same values (lanes 4, 2 and 1 apart, then within the lane).
+__device__ __forceinline__ void quantize_block_q8_1_lanes(const float *src, int k0, int in_dim, int j, uint32_t *out,
+                                                          bool raw) {
+    float v[4];
+    if (k0 + 4 <= in_dim) {
+        __builtin_memcpy(v, src + k0, sizeof(v));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = k0 + e < in_dim ? src[k0 + e] : 0.0f;
+    }
+    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    amax = fmaxf(amax, dpp_move<0xb1>(amax));
+    amax = fmaxf(amax, dpp_move<0x4e>(amax));
+    amax = fmaxf(amax, dpp_move<0x141>(amax));
+    const float d = amax > 0.0f ? amax / 127.0f : 0.0f;
+    const float id = d > 0.0f ? 1.0f / d : 0.0f;
+    uint32_t word = 0;
+    int qsum = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        int q = static_cast<int>(rintf(__fmul_rn(v[e], id)));
+        q = q < -127 ? -127 : (q > 127 ? 127 : q);
+        qsum += q;
+        word |= (static_cast<uint32_t>(q) & 0xffu) << (8 * e);
+    }
+    out[1 + j] = word;
+    float sum;
+    if (raw) {  // uniform
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += __shfl_xor(v[e], off, 64);
+        sum = (v[0] + v[2]) + (v[1] + v[3]);
+    } else {
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1) qsum += __shfl_xor(qsum, off, 64);
+        sum = __fmul_rn(d, static_cast<float>(qsum));
+    }
+    if (j == 0) *out = f32_to_f16_bits(d) | (f32_to_f16_bits(sum) << 16);
+}
+
 // Block qb of a weight row against activation block (dx, sx, qx[32]).
 template <int T>
 __device__ __forceinline__ float block_dot_q8_1(const uint8_t *row, int qb, float dx, float sx, const int8_t *qx) {

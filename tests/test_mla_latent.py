@@ -264,3 +264,40 @@ def test_context_v(T, pos):
     out = empty_f32(NH, VH)
     qlin.call("qlin_launch_mla_absorb_context_v_device_pos", dev(s), dev(kvb), out, NH, QN, VH, _pos(pos), T)
     assert normwise_rel_err(host(out), orc.mla_absorb_context_v(s, kvb, NH, QN, VH, pos, T)) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_lora,qk_rope,T,pos", [(72, 20, 70, 69),       # a partial block, a partial rope chunk
+                                                   (96, 12, 300, 299),     # three blocks: an odd one in the column pair
+                                                   (512, 64, 2304, 2303),  # more positions than one round of scores
+                                                   (544, 64, 40, 17),      # more blocks than the block form of attend takes
+                                                   (96, 12, 33, -1)])      # no positions
+def test_latent_shapes(kv_lora, qk_rope, T, pos):
+    """Scores, context and attend at shapes off DeepSeek's, each against the oracle (1e-5 normwise, as above)."""
+    from gpu_util import banner, bind_stream, dev, empty_f32, host
+    nh, qn = 3, 16
+    kv, cache, crb = make_cache(T, kv_lora, qk_rope, 140 + kv_lora)
+    rng = np.random.default_rng(141 + T)
+    nb = -(-kv_lora // 32)
+    q_abs = rng.standard_normal((nh, kv_lora)).astype(np.float32) * 0.05
+    q = rng.standard_normal((nh, qn + qk_rope)).astype(np.float32) * 0.5
+    delta = rng.standard_normal((nh, nb)).astype(np.float32)
+    banner(f"mla shapes kv_lora={kv_lora} rope={qk_rope} T={T} pos={pos}")
+    bind_stream()
+    sd, lat_d, dl_d = dev(np.full((nh, T), -7.0, np.float32)), empty_f32(nh, kv_lora), empty_f32(nh, nb)
+    cd, kd = dev(cache), dev(kv)
+    qlin.call("qlin_launch_mla_absorb_scores_device_pos", dev(q_abs), dev(q), cd, crb, dev(delta), kd, sd, nh, qn,
+              qk_rope, kv_lora, _pos(pos), T, SCALE)
+    qlin.call("qlin_launch_mla_absorb_context_device_pos", sd, cd, crb, dl_d, lat_d, nh, kv_lora, _pos(pos), T)
+    got, lat, dl = host(sd), host(lat_d), host(dl_d)
+    qlin.call("qlin_launch_mla_absorb_attend_device_pos", dev(q_abs), dev(q), cd, crb, dev(delta), dl_d, kd, lat_d, nh,
+              qn, qk_rope, kv_lora, _pos(pos), T, SCALE)
+    if pos < 0:
+        assert (got == -7.0).all() and not lat.any() and not dl.any() and not host(lat_d).any()
+        return
+    ref = orc.mla_absorb_scores(q_abs, q, cache, crb, delta, kv, nh, qn, qk_rope, kv_lora, pos, T, SCALE)
+    assert normwise_rel_err(got[:, :pos + 1], ref[:, :pos + 1]) <= 1e-5
+    rlat, rdl = orc.mla_absorb_context(got, cache, crb, nh, kv_lora, pos, T)
+    assert normwise_rel_err(lat, rlat) <= 1e-5 and normwise_rel_err(dl, rdl) <= 1e-5
+    rlat, rdl = orc.mla_absorb_attend(q_abs, q, cache, crb, delta, kv, nh, qn, qk_rope, kv_lora, pos, T, SCALE)
+    assert normwise_rel_err(host(lat_d), rlat) <= 1e-5 and normwise_rel_err(host(dl_d), rdl) <= 1e-5
