@@ -9,19 +9,19 @@
 // (q4k_rows_dot, qlin_rows.hpp): the nibble q enters as the exact bf16 128 + q and x as the bf16 pair
 // hi = bf16(x), lo = bf16(x - hi), so every product is exact and accumulates in f32; per sub-block
 // and 16-token tile one MFMA pair gives sum x (128 + q) for 16 weight rows and another pair sum x,
-// and two fmas per output apply the scales.  The other formats multiply the canonical f32 element values (decoded as the
-// reference decodes them) on v_mfma_f32_16x16x4_f32: the contraction the reference runs one warp
-// per (r, o), with the same f32 operands and only the summation order changed.
+// and two fmas per output apply the scales.  The other formats: rows_kernel, below.
 //
-// Layout.  A workgroup owns a tile of 16 output rows and all of K; its 8 waves take the chunks of K in
-// turn (wave w: w, w + 8, ...; Q4_K super-blocks, eight 32-element blocks otherwise).  Lane l supplies output row l % 16 and token l % 16 of the current
-// 16-token tile, and k-slots of group g = l / 16 of each MFMA (Q4_K: elements 8g .. 8g+7 of a
-// sub-block).  D holds tokens 4g .. 4g+3 of row l % 16.  The waves' partials meet in LDS and are
-// summed in wave order.  A grid row per 64 tokens.
+// Layout (Q4_K).  A workgroup owns a tile of 16 output rows and all of K; its 8 waves take the
+// super-blocks in turn (wave w: w, w + 8, ...).  Lane l supplies output row l % 16 and token l % 16 of the
+// current 16-token tile, and elements 8g .. 8g+7 of each sub-block (g = l / 16).  D holds tokens 4g ..
+// 4g+3 of row l % 16.  The waves' partials meet in LDS and are summed in wave order.  A grid row per 64
+// tokens.
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
 #include "qlin_mfma.hpp"
 #include "qlin_rows.hpp"
+#include "qlin_values8.hpp"
+#include <type_traits>
 
 namespace qlin {
 namespace {
@@ -170,157 +170,456 @@ __global__ __launch_bounds__(kDThreads) void q4k_dense_kernel(const DenseArgs a)
     }
 }
 
-// 8 bytes at a 2-byte aligned address, as two dwords.
-__device__ __forceinline__ void ld8_a2(const uint8_t *p, uint32_t &lo, uint32_t &hi) {
-    const uint16_t *h = reinterpret_cast<const uint16_t *>(p);
-    lo = h[0] | (static_cast<uint32_t>(h[1]) << 16);
-    hi = h[2] | (static_cast<uint32_t>(h[3]) << 16);
+// ---- the other formats (Q4_0, Q5_0, Q8_0, Q6_K) --------------------------------------------------
+//
+// v_mfma_f32_16x16x32_f16 with the tokens as the MFMA rows, the operands of the prefill GEMM
+// (qlin_gemm.hip): B = q less its offset (Q6_K: sc (q - 32) in two exact parts), A = x 2^s split into fp16
+// hi and lo, s per token from its largest magnitude so far (rescaled when a value 8 times that comes).
+// Nothing is shared between waves: each takes whole units of four 32-blocks of K in turn (wave w: w, w + 8,
+// ...) for all of the workgroup's rows and tokens, straight from memory, one unit's weights and one token
+// tile's x ahead, so short and narrow products need no barrier per step; the waves' sums meet in LDS.
+// What bounds it: a tile's chain (x turned in LDS, its scale, 64 split and 16-32 scaling instructions
+// around 8-16 MFMAs) with two waves on a SIMD.  A request whose lanes lie in different rows costs the
+// address path a cycle per lane, which is why x is read along its rows and a lane group reads a whole
+// block.  Against f32 matrix cores (v_mfma_f32_16x16x4_f32) on decoded values with the layout's own
+// 8-byte pieces: Q6_K [3584, 18944] at 12 rows 78 -> 33 us, Q5_0 [4096, 4096] at 6 rows 19 -> 10 us, Q8_0
+// [4096, 4096] at 100 rows 108 -> 38 us, Q5_0 [30000, 1024] at 40 rows 92 -> 26 us.
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f32x4 mfma_h(const uint4 &a, const uint4 &b, const f32x4 &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ uint32_t byte_of(uint32_t lo, uint32_t hi, int i) {
-    return ((i < 4 ? lo : hi) >> (8 * (i & 3))) & 0xffu;
+__device__ __forceinline__ uint32_t h2u(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
+__device__ __forceinline__ f16x2 u2h(uint32_t u) { return __builtin_bit_cast(f16x2, u); }
+__device__ __forceinline__ f16x2 splat(float v) {
+    const _Float16 h = static_cast<_Float16>(v);
+    return f16x2{h, h};
+}
+// the fp16 pairs 1024 + byte of bytes 0, 1 and 2, 3
+__device__ __forceinline__ f16x2 bytes_lo(uint32_t v) { return u2h(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)); }
+__device__ __forceinline__ f16x2 bytes_hi(uint32_t v) { return u2h(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)); }
+__device__ __forceinline__ uint4 minus8(uint32_t a, uint32_t b, f16x2 off) {
+    return make_uint4(h2u(bytes_lo(a) + off), h2u(bytes_hi(a) + off), h2u(bytes_lo(b) + off), h2u(bytes_hi(b) + off));
+}
+__device__ __forceinline__ uint32_t bit4_of_bytes(uint32_t b) { return (__umul24(b & 0xfu, 0x204081u) & 0x01010101u) << 4; }
+
+constexpr int kUnit = 4;  // 32-blocks of a unit
+
+// Lane moves between the four groups of 16 lanes (rows) of a wave.
+// swap32(a, b): a = {a's rows 0, 1, b's rows 0, 1}, b = {a's rows 2, 3, b's rows 2, 3}
+__device__ __forceinline__ void swap32(uint32_t &a, uint32_t &b) {
+    const auto s = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = static_cast<uint32_t>(s[0]);
+    b = static_cast<uint32_t>(s[1]);
+}
+// swap16(a, b): a = {a0, b0, a2, b2}, b = {a1, b1, a3, b3} by rows
+__device__ __forceinline__ void swap16(uint32_t &a, uint32_t &b) {
+    const auto s = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = static_cast<uint32_t>(s[0]);
+    b = static_cast<uint32_t>(s[1]);
+}
+// o[j] = group j's v, in every group
+__device__ __forceinline__ void all_groups(uint32_t v, uint32_t (&o)[4]) {
+    uint32_t lo = v, hi = v;
+    swap32(lo, hi);
+    o[0] = o[1] = lo;
+    swap16(o[0], o[1]);
+    o[2] = o[3] = hi;
+    swap16(o[2], o[3]);
 }
 
-// Elements k0 .. k0+7 of a row (k0 a multiple of 8: one block, one scale group), canonical values
-// as the per-element decoders give them (kernel.cu:1122-1185, ggml's Q4_0): the raw words first
-// (so that a wave can have several blocks' loads in flight), then the values.
+// A unit of one row, loaded with a whole block per lane group (as few, wide requests as the layout of one
+// row per lane allows: each costs the address path a cycle per lane), then exchanged between the groups
+// so that group g holds elements 8g .. 8g+7 of every block.  blk: the unit's first block; last: the row's
+// last block (a unit cut short reads it again).
 template <int T>
-__device__ __forceinline__ void raw8(const uint8_t *row, int k0, uint32_t (&w)[5]) {
-    if constexpr (T == T_Q8_0) {
-        const uint8_t *b = row + static_cast<size_t>(k0 >> 5) * 34;
-        w[0] = ld_u16(b);
-        ld8_a2(b + 2 + (k0 & 31), w[1], w[2]);
-    } else if constexpr (T == T_Q4_0 || T == T_Q5_0) {
-        constexpr int BB = T == T_Q4_0 ? 18 : 22, QS = T == T_Q4_0 ? 2 : 6;
-        const uint8_t *b = row + static_cast<size_t>(k0 >> 5) * BB;
-        w[0] = ld_u16(b);
-        ld8_a2(b + QS + (k0 & 15), w[1], w[2]);
-        if constexpr (T == T_Q5_0) w[3] = ld_u16(b + 2) | (ld_u16(b + 4) << 16);
-    } else {  // Q6_K: half h, group g of 32, lanes l0 .. l0+7 (one 16-element scale)
-        const uint8_t *b = row + static_cast<size_t>(k0 >> 8) * 210;
-        const int e = k0 & 255, half = e >> 7, grp = (e & 127) >> 5, l0 = e & 31;
-        ld8_a2(b + half * 64 + l0 + 32 * (grp & 1), w[0], w[1]);
-        ld8_a2(b + 128 + half * 32 + l0, w[2], w[3]);
-        w[4] = ld_u16(b + 208) | (static_cast<uint32_t>(b[192 + half * 8 + l0 / 16 + 2 * grp]) << 16);
-    }
-}
-
-template <int T>
-__device__ __forceinline__ void values8(const uint32_t (&w)[5], int k0, float (&v)[8]) {
-    if constexpr (T == T_Q8_0) {
-        const float d = f16_bits_to_f32(w[0]);
+struct Unit {
+    static constexpr int W = T == T_Q8_0 ? 8 : 4;
+    uint32_t q[W], d, qh;
+    __device__ __forceinline__ void load(const uint8_t *row, int blk, int last, int g) {
+        const uint8_t *b = row + static_cast<size_t>(min(blk + g, last)) * Block<T>::bytes;
+        d = ld_u16(b);
+        if constexpr (T == T_Q5_0) qh = ld4_a2(b + 2);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = mul_rn(d, static_cast<float>(static_cast<int8_t>(byte_of(w[1], w[2], i))));
-    } else if constexpr (T == T_Q4_0 || T == T_Q5_0) {
-        const int e0 = k0 & 31, sh = e0 >= 16 ? 4 : 0;
-        const float d = f16_bits_to_f32(w[0]);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            int q = static_cast<int>((byte_of(w[1], w[2], i) >> sh) & 15u);
-            if constexpr (T == T_Q5_0) q |= static_cast<int>(((w[3] >> (e0 + i)) & 1u) << 4);
-            v[i] = mul_rn(d, static_cast<float>(q - (T == T_Q4_0 ? 8 : 16)));
-        }
-    } else {
-        const int grp = ((k0 & 255) & 127) >> 5;
-        const int sc = static_cast<int8_t>(w[4] >> 16);
-        const float dsc = mul_rn(f16_bits_to_f32(w[4] & 0xffffu), static_cast<float>(sc));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t lb = byte_of(w[0], w[1], i), hb = byte_of(w[2], w[3], i);
-            const int q = static_cast<int>(((grp < 2 ? lb : lb >> 4) & 15u) | (((hb >> (2 * grp)) & 3u) << 4)) - 32;
-            v[i] = mul_rn(dsc, static_cast<float>(q));
+        for (int i = 0; i < W; i += 4) {
+            const u32x4 v = ld16_a2(b + (T == T_Q5_0 ? 6 : 2) + 4 * i);
+            q[i] = v.x;
+            q[i + 1] = v.y;
+            q[i + 2] = v.z;
+            q[i + 3] = v.w;
         }
     }
-}
-
-// The other formats (Q4_0, Q5_0, Q8_0, Q6_K): the waves take 32-element blocks in turn (wave w: w,
-// w + 8, ...); a lane's 8 values of a block are decoded once and serve every token tile.
-template <int T, int MODE>
-__global__ __launch_bounds__(kDThreads) void dense_generic_kernel(const DenseArgs a) {
-    constexpr int NW = MODE == kSwiGLU ? 2 : 1;
-    __shared__ f32x4 part[kDWaves][NW][1][64];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n = lane & 15, g = lane >> 4;
-    const int K = a.k, nb32 = K / 32;
-    const int row0 = blockIdx.x * 16;
-    const int row = min(row0 + n, a.n - 1);
-    const int t0 = blockIdx.y * 16;  // one 16-token tile per grid row
-    constexpr int ntt = 1;
-    const uint8_t *rp[2] = {a.w0 + static_cast<size_t>(row) * a.rb, a.w1 + static_cast<size_t>(row) * a.rb};
-    const float *xrow = a.x + static_cast<size_t>(min(t0 + n, a.m - 1)) * K;  // past m: the last token
-
-    f32x4 D[NW][1];
+    // the operands and scales of the unit's blocks
+    __device__ __forceinline__ void operands(int g, uint4 (&b)[kUnit], uint4 (&)[1], float (&dw)[kUnit]) const {
+        uint32_t ds[4], o[kUnit][2];
+        all_groups(d, ds);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) D[w][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // groups of U consecutive blocks, wave w: groups w, w + 8, ...; a group's weight words and
-    // activations are all requested before its first block is used
-    constexpr int U = 4;
-    for (int b0 = wave * U; b0 < nb32; b0 += kDWaves * U) {
-        uint32_t raw[NW][U][5];
-        float4 xq[U][2];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k0 = 32 * min(b0 + u, nb32 - 1) + 8 * g;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) raw8<T>(rp[w], k0, raw[w][u]);
-            xq[u][0] = *reinterpret_cast<const float4 *>(xrow + k0);
-            xq[u][1] = *reinterpret_cast<const float4 *>(xrow + k0 + 4);
+        for (int e = 0; e < 2; ++e) {  // the dwords of a lane's 8 bytes
+            if constexpr (T == T_Q8_0) {
+                uint32_t m0 = q[e], m1 = q[2 + e], m2 = q[4 + e], m3 = q[6 + e];
+                swap32(m0, m2);
+                swap32(m1, m3);
+                swap16(m0, m1);
+                swap16(m2, m3);
+                o[0][e] = m0;
+                o[1][e] = m1;
+                o[2][e] = m2;
+                o[3][e] = m3;
+            } else {  // bytes 8 (g & 1) .. + 7 of every block
+                uint32_t m0 = q[e], m1 = q[2 + e];
+                swap16(m0, m1);
+                uint32_t a0 = m0, a2 = m0, a1 = m1, a3 = m1;
+                swap32(a0, a2);
+                swap32(a1, a3);
+                o[0][e] = a0;
+                o[1][e] = a1;
+                o[2][e] = a2;
+                o[3][e] = a3;
+            }
         }
-        __builtin_amdgcn_sched_barrier(0);  // keep the group's loads ahead of its first use
-        // straight-line over the group (no branch lets the compiler sink a load to its use): a block
-        // past the end repeats the last one with zero activations
+        [[maybe_unused]] uint32_t h[4];
+        if constexpr (T == T_Q5_0) all_groups(qh, h);
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool in = b0 + u < nb32;
-            const int k0 = 32 * min(b0 + u, nb32 - 1) + 8 * g;
-            const float xv[8] = {in ? xq[u][0].x : 0.0f, in ? xq[u][0].y : 0.0f, in ? xq[u][0].z : 0.0f,
-                                 in ? xq[u][0].w : 0.0f, in ? xq[u][1].x : 0.0f, in ? xq[u][1].y : 0.0f,
-                                 in ? xq[u][1].z : 0.0f, in ? xq[u][1].w : 0.0f};
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                float v[8];
-                values8<T>(raw[w][u], k0, v);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) D[w][0] = mfma_f32(xv[i], v[i], D[w][0]);
+        for (int j = 0; j < kUnit; ++j) {
+            dw[j] = f16_bits_to_f32(ds[j]);
+            if constexpr (T == T_Q8_0) {
+                b[j] = minus8(o[j][0] ^ 0x80808080u, o[j][1] ^ 0x80808080u, splat(-1152.0f));
+            } else {  // low nibbles: elements 0..15, high: 16..31
+                uint32_t u = (o[j][0] >> (4 * (g >> 1))) & 0x0f0f0f0fu, v = (o[j][1] >> (4 * (g >> 1))) & 0x0f0f0f0fu;
+                if constexpr (T == T_Q5_0) {
+                    const uint32_t hb = h[j] >> (8 * g);
+                    u |= bit4_of_bytes(hb);
+                    v |= bit4_of_bytes(hb >> 4);
+                }
+                b[j] = minus8(u, v, splat(T == T_Q5_0 ? -1040.0f : -1032.0f));
             }
         }
     }
-
+};
+template <>
+struct Unit<T_Q6_K> {  // half a super-block
+    uint2 l[2], h, sc;
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t *row, int blk, int, int g) {
+        const uint8_t *sb = row + static_cast<size_t>(blk >> 3) * 210;
+        const int half = (blk >> 2) & 1;
+        l[0] = ld8_a2(sb + 64 * half + 8 * g);
+        l[1] = ld8_a2(sb + 64 * half + 32 + 8 * g);
+        h = ld8_a2(sb + 128 + 32 * half + 8 * g);
+        sc = ld8_a2(sb + 192 + 8 * half);
+        d = ld_u16(sb + 208);
+    }
+    __device__ __forceinline__ void operands(int g, uint4 (&b1)[kUnit], uint4 (&b2)[kUnit], float (&dw)[kUnit]) const {
+        dw[0] = f16_bits_to_f32(d);
 #pragma unroll
-    for (int w = 0; w < NW; ++w)
+        for (int j = 0; j < kUnit; ++j) operand(j, g, b1[j], b2[j]);
+    }
+    __device__ __forceinline__ void operand(int j, int g, uint4 &b1, uint4 &b2) const {
+        const uint32_t s = (((j < 2 ? sc.x : sc.y) >> (8 * (2 * (j & 1) + (g >> 1)))) & 0xffu) ^ 0x80u;
+        const f16x2 s2 = u2h(0x64006400u | s | (s << 16)) + splat(-1152.0f);
+        const uint2 lw = l[j & 1];
+        const uint32_t u = ((lw.x >> (4 * (j >> 1))) & 0x0f0f0f0fu) | (((h.x >> (2 * j)) & 0x03030303u) << 4);
+        const uint32_t v = ((lw.y >> (4 * (j >> 1))) & 0x0f0f0f0fu) | (((h.y >> (2 * j)) & 0x03030303u) << 4);
+        const uint4 q = minus8(u, v, splat(-1056.0f));
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        uint32_t p1[4], p2[4];
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt)
-            if (tt < ntt) part[wave][w][tt][lane] = D[w][tt];
-    __syncthreads();
-    const int rows = min(16, a.n - row0);
-    for (int i = tid; i < ntt * 256; i += kDThreads) {
-        const int tl = i >> 4, o = i & 15;
-        const int t = t0 + tl;
-        if (o >= rows || t >= a.m) continue;
-        const int tt = tl >> 4, l = ((tl & 15) >> 2) * 16 + o, r = tl & 3;
-        float v0 = 0.0f, v1 = 0.0f;
-        for (int wv = 0; wv < kDWaves; ++wv) {
-            v0 += part[wv][0][tt][l][r];
-            if constexpr (NW == 2) v1 += part[wv][NW - 1][tt][l][r];
+        for (int e = 0; e < 4; ++e) {
+            const f16x2 p = u2h(w[e]) * s2;
+            p1[e] = h2u(p);
+            p2[e] = h2u(__builtin_elementwise_fma(u2h(w[e]), s2, -p));
         }
-        float *yo = a.y + static_cast<size_t>(t) * a.n + row0 + o;
+        b1 = make_uint4(p1[0], p1[1], p1[2], p1[3]);
+        b2 = make_uint4(p2[0], p2[1], p2[2], p2[3]);
+    }
+};
+
+// max over the four lane groups of v (>= 0, whose bits order as it does): every lane gets its token's
+__device__ __forceinline__ float max_over_groups(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    const uint32_t c = max(static_cast<uint32_t>(s[0]), static_cast<uint32_t>(s[1]));
+    const auto t = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+    return __builtin_bit_cast(float, max(static_cast<uint32_t>(t[0]), static_cast<uint32_t>(t[1])));
+}
+__device__ __forceinline__ float max3_abs(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// hi and lo fp16 parts of 8 values times sc (a power of two)
+__device__ __forceinline__ void split8(const f32x4 &a, const f32x4 &b, float sc, uint4 &hi, uint4 &lo) {
+    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = h2u(f16x2{static_cast<_Float16>(fmaf(v[2 * i], sc, 0.0f)), static_cast<_Float16>(fmaf(v[2 * i + 1], sc, 0.0f))});
+        asm("" : "+v"(h[i]));  // one packed value (its halves would otherwise be formed twice)
+        const f16x2 hp = u2h(h[i]);
+        l[i] = h2u(f16x2{static_cast<_Float16>(fmaf(v[2 * i], sc, -static_cast<float>(hp[0]))),
+                         static_cast<_Float16>(fmaf(v[2 * i + 1], sc, -static_cast<float>(hp[1])))});
+    }
+    hi = make_uint4(h[0], h[1], h[2], h[3]);
+    lo = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+// an infinite value has no lo part
+__device__ __forceinline__ uint32_t finite_lo(uint32_t h, uint32_t l) {
+    l = (h & 0x7fffu) == 0x7c00u ? l & 0xffff0000u : l;
+    return (h & 0x7fff0000u) == 0x7c000000u ? l & 0x0000ffffu : l;
+}
+__device__ __forceinline__ void drop_inf(const uint4 &h, uint4 &l) {
+    l = make_uint4(finite_lo(h.x, l.x), finite_lo(h.y, l.y), finite_lo(h.z, l.z), finite_lo(h.w, l.w));
+}
+
+template <int T, int MODE, int NT, int TT>
+__global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
+    static_assert(MODE != kSwiGLU || NT % 2 == 0, "gate and up tiles in pairs");
+    constexpr int OT = MODE == kSwiGLU ? NT / 2 : NT;  // output row tiles
+    constexpr bool Q6 = T == T_Q6_K;
+    extern __shared__ f32x4 part[];  // [wave][row tile][token tile][lane]
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = lane & 15, g = lane >> 4;
+    const int K = a.k, nblk = K / 32, nunit = (nblk + kUnit - 1) / kUnit;
+    int bx, by;
+    gemm_tile((a.n + 16 * OT - 1) / (16 * OT), (a.m + 16 * TT - 1) / (16 * TT), bx, by);
+    const int row0 = bx * 16 * OT, t0 = by * 16 * TT;
+
+    const uint8_t *rp[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const size_t row = min(row0 + (t % OT) * 16 + n, a.n - 1);
+        rp[t] = (t < OT ? a.w0 : a.w1) + row * a.rb;
+    }
+    f32x4 acc[TT][NT];
+    float limit[TT];  // 2^(15 - s) of the lane's token in each tile (0: no value yet)
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+        limit[i] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    // x of a token tile's unit: read along the tokens' rows (32 lanes of a token, two tokens a request),
+    // turned in the wave's own LDS (slot c of token t at c ^ t) into lane (token n, elements 8g .. 8g+7 of
+    // every block).  A wave's LDS accesses complete in order, so it needs no waits of its own.
+    f32x4 *turn = part + wave * (16 * 8 * kUnit);
+    const int lt = lane >> 5, lc = lane & 31;
+    auto load_x = [&](f32x4 (&x)[2 * kUnit], int i, int u) {
+        // a unit cut short reads the row's last block again
+        const int c = min(8 * kUnit * u + lc, 8 * nblk - 8 + (lc & 7));
+#pragma unroll
+        for (int p = 0; p < 2 * kUnit; ++p)
+            x[p] = reinterpret_cast<const f32x4 *>(a.x + static_cast<size_t>(min(t0 + 16 * i + 2 * p + lt, a.m - 1)) * K)[c];
+    };
+    auto turn_x = [&](const f32x4 (&x)[2 * kUnit], f32x4 (&r)[2 * kUnit]) {
+#pragma unroll
+        for (int p = 0; p < 2 * kUnit; ++p) turn[(2 * p + lt) * 32 + (lc ^ (2 * p + lt))] = x[p];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int e = 0; e < 2 * kUnit; ++e) r[e] = turn[n * 32 + ((8 * (e >> 1) + 2 * g + (e & 1)) ^ n)];
+        __builtin_amdgcn_wave_barrier();
+    };
+    Unit<T> raw[NT];
+    f32x4 ahead[2 * kUnit];
+    int u = wave;
+    if (u < nunit) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) raw[t].load(rp[t], kUnit * u, nblk - 1, g);
+        load_x(ahead, 0, u);
+    }
+    for (; u < nunit; u += kDWaves) {  // uniform
+        uint4 B[NT][kUnit], B2[NT][Q6 ? kUnit : 1];
+        float dw[NT][kUnit];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) raw[t].operands(g, B[t], B2[t], dw[t]);
+        const int next = u + kDWaves;
+        auto tile = [&](int i) {
+            f32x4 x[2 * kUnit];
+            turn_x(ahead, x);
+            // the next tile's x (of this unit or the next); the next unit's weights behind the first tile's
+            __builtin_amdgcn_sched_barrier(0);
+            if (i + 1 < TT) load_x(ahead, i + 1, u);
+            else if (next < nunit) load_x(ahead, 0, next);
+            if (i == 0 && next < nunit) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) raw[t].load(rp[t], kUnit * next, nblk - 1, g);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (!Q6 && kUnit * u + kUnit > nblk) {  // uniform: a unit cut short
+                asm volatile("");
+#pragma unroll
+                for (int j = 1; j < kUnit; ++j)
+                    if (kUnit * u + j >= nblk) x[2 * j] = x[2 * j + 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            float am = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 2 * kUnit; ++e) am = max3_abs(x[e][2], x[e][3], max3_abs(x[e][0], x[e][1], am));
+            am = max_over_groups(am);
+            const bool inf = !(am <= 3.4e38f);
+            if (__any(am > limit[i])) {  // uniform, rare: new scales, the sums so far brought to them
+                asm volatile("");
+                float f = 1.0f;
+                if (am > limit[i]) {
+                    if (inf) {
+                        if (limit[i] == 0.0f) limit[i] = 32768.0f;
+                    } else {
+                        int ex;
+                        (void)frexpf(am, &ex);
+                        const float was = limit[i];
+                        limit[i] = ldexpf(1.0f, 15 - min(13 - ex, 120));
+                        if (was > 0.0f) f = was / limit[i];
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float fr = __shfl(f, 4 * g + r, 64);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) acc[i][t][r] *= fr;
+                }
+            }
+            // 2^s: the exponents of limit and 2^s add up to 15 (no value yet: some finite number, against zeros)
+            const float sc = __builtin_bit_cast(float, (269u << 23) - __builtin_bit_cast(uint32_t, limit[i]));
+            auto blocks = [&](auto with_inf) {
+                [[maybe_unused]] f32x4 D6[NT];
+#pragma unroll
+                for (int j = 0; j < kUnit; ++j) {
+                    uint4 hi, lo;
+                    split8(x[2 * j], x[2 * j + 1], sc, hi, lo);
+                    uint4 hi2 = hi;  // against B2, which may be 0 where the weight is not: no infinite values
+                    if constexpr (decltype(with_inf)::value) {
+                        drop_inf(hi, lo);
+                        drop_inf(hi, hi2);
+                    }
+                    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (Q6) {  // d is the unit's: its blocks add up first
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) D6[t] = mfma_h(hi, B[t][j], j ? D6[t] : zero);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) D6[t] = mfma_h(hi2, B2[t][j], D6[t]);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) D6[t] = mfma_h(lo, B[t][j], D6[t]);
+                    } else {
+                        f32x4 D[NT];
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) D[t] = mfma_h(hi, B[t][j], zero);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) D[t] = mfma_h(lo, B[t][j], D[t]);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][j], D[t][r], acc[i][t][r]);
+                    }
+                }
+                if constexpr (Q6) {
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][0], D6[t][r], acc[i][t][r]);
+                }
+            };
+            if (__any(inf)) blocks(std::true_type{});  // uniform
+            else blocks(std::false_type{});
+#pragma unroll
+            for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(acc[i][t]));  // (not sunk below the next tile)
+        };
+        tile(0);
+        if constexpr (TT > 1) tile(1);
+        if constexpr (TT > 2) {
+            tile(2);
+            tile(3);
+        }
+    }
+    __syncthreads();  // (the sums below take the LDS of the tiles)
+
+    // each wave's sums at their true scale; lane (row, g) of D holds tokens 4g .. 4g+3
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+        const float inv = limit[i] > 0.0f ? limit[i] * 0x1p-15f : 1.0f;
+        f32x4 iv;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) iv[r] = __shfl(inv, 4 * g + r, 64);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) part[((wave * NT + t) * TT + i) * 64 + lane] = acc[i][t] * iv;
+    }
+    __syncthreads();
+    const int rows = min(16 * OT, a.n - row0), toks = min(16 * TT, a.m - t0);
+    for (int e = tid; e < 16 * OT * 16 * TT; e += kDThreads) {
+        const int tl = e / (16 * OT), o = e % (16 * OT);
+        if (o >= rows || tl >= toks) continue;
+        const int i = tl >> 4, t = o >> 4, l = ((tl & 15) >> 2) * 16 + (o & 15), r = tl & 3;
+        float v0 = 0.0f, v1 = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kDWaves; ++w) {
+            v0 += part[((w * NT + t) * TT + i) * 64 + l][r];
+            if constexpr (MODE == kSwiGLU) v1 += part[((w * NT + OT + t) * TT + i) * 64 + l][r];
+        }
+        float *yo = a.y + static_cast<size_t>(t0 + tl) * a.n + row0 + o;
         if constexpr (MODE == kSwiGLU) *yo = v0 / (1.0f + expf(-v0)) * v1;
-        else if constexpr (MODE == kAdd) add_out(a, yo, t, row0 + o, v0);
+        else if constexpr (MODE == kAdd) add_out(a, yo, t0 + tl, row0 + o, v0);
         else *yo = v0;
+    }
+}
+
+template <int T, int MODE, int NT, int TT>
+hipError_t launch_rows(const DenseArgs &a, hipStream_t s) {
+    constexpr int OT = MODE == kSwiGLU ? NT / 2 : NT;
+    const auto max = [](int a, int b) { return a > b ? a : b; };
+    const dim3 grid = gemm_grid((a.n + 16 * OT - 1) / (16 * OT), (a.m + 16 * TT - 1) / (16 * TT));
+    hipLaunchKernelGGL((rows_kernel<T, MODE, NT, TT>), grid, dim3(kDThreads), sizeof(f32x4) * kDWaves * max(NT * TT * 64, 16 * 8 * kUnit), s, a);
+    return hipGetLastError();
+}
+
+// The tiles of a launch: NT row tiles (of a SwiGLU: NT / 2 outputs') by TT token tiles per workgroup, one
+// workgroup on a CU at a time.  Measured, a round of workgroups takes about 2 us plus, per unit of a wave,
+// 2.1 (1 x 1), 3.3 (2 x 1), 3.2 (1 x 2), 4.6 (2 x 2) and 8.8 us (2 x 4): larger tiles split x and read the
+// weights for more products, smaller ones fill the chip.  The cheapest total is taken.
+struct RowsPlan {
+    int nt, tt;
+    float us;
+};
+RowsPlan rows_plan(int n, int k, int m, bool swiglu) {
+    static constexpr struct {
+        int nt, tt;
+        float unit;
+    } kinds[] = {{1, 1, 2.1f}, {2, 1, 3.3f}, {1, 2, 3.2f}, {2, 2, 4.6f}, {2, 4, 8.8f}};
+    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+    const float units = static_cast<float>((k / 32 + kUnit * kDWaves - 1) / (kUnit * kDWaves));
+    RowsPlan best{0, 0, 0.0f};
+    for (const auto &c : kinds) {
+        if (swiglu && c.nt == 1) continue;
+        const int rows = 16 * c.nt / (swiglu ? 2 : 1), toks = 16 * c.tt;
+        const int64_t wgs = static_cast<int64_t>((n + rows - 1) / rows) * ((m + toks - 1) / toks);
+        const float us = static_cast<float>((wgs + cus - 1) / cus) * (2.0f + units * c.unit);
+        if (!best.nt || us < best.us) best = RowsPlan{c.nt, c.tt, us};
+    }
+    return best;
+}
+
+template <int T, int MODE>
+hipError_t by_shape(const DenseArgs &a, hipStream_t s) {
+    const RowsPlan p = rows_plan(a.n, a.k, a.m, MODE == kSwiGLU);
+    if constexpr (MODE != kSwiGLU) {
+        if (p.nt == 1) return p.tt == 1 ? launch_rows<T, MODE, 1, 1>(a, s) : launch_rows<T, MODE, 1, 2>(a, s);
+    }
+    switch (p.tt) {
+        case 1: return launch_rows<T, MODE, 2, 1>(a, s);
+        case 2: return launch_rows<T, MODE, 2, 2>(a, s);
+        default: return launch_rows<T, MODE, 2, 4>(a, s);
     }
 }
 
 template <int T>
 hipError_t launch_dense(const DenseArgs &a, int mode, hipStream_t s) {
-    const dim3 grid((a.n + 15) / 16, (a.m + 15) / 16);
     switch (mode) {
-        case kStore: hipLaunchKernelGGL((dense_generic_kernel<T, kStore>), grid, dim3(kDThreads), 0, s, a); break;
-        case kAdd: hipLaunchKernelGGL((dense_generic_kernel<T, kAdd>), grid, dim3(kDThreads), 0, s, a); break;
-        case kSwiGLU: hipLaunchKernelGGL((dense_generic_kernel<T, kSwiGLU>), grid, dim3(kDThreads), 0, s, a); break;
+        case kStore: return by_shape<T, kStore>(a, s);
+        case kAdd: return by_shape<T, kAdd>(a, s);
+        case kSwiGLU: return by_shape<T, kSwiGLU>(a, s);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 }  // namespace
@@ -332,6 +631,8 @@ bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const f
     // the per-element decoder reads 16-bit fields: 2-byte aligned blocks
     return k % 32 == 0 && rb % 2 == 0 && al(w0, 2) && (!w1 || al(w1, 2)) && al(x, 16);
 }
+
+float dense_us(int n, int k, int m, bool swiglu) { return rows_plan(n, k, m, swiglu).us; }
 
 hipError_t dense_matmul(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const float *x, float *y, int n,
                         int k, int m, int mode, hipStream_t s, const RouteCombine *combine) {

@@ -86,7 +86,16 @@ hipError_t gemv(int type, const uint8_t *w, size_t rb, const float *x, float *y,
         return mfma_gemv(type, &w, &y, &n, 1, rb, x, k, add, s);
     if (type == T_Q4_K && m == 1 && q4k_stream_ok(&w, 1, rb, x, n, k, false))
         return q4k_stream_gemv(&w, &y, &n, 1, rb, x, k, add, s);
-    if (m >= kF32GemmMinRows && f32_gemm_ok(type, w, rb, x, k)) return f32_gemm(type, w, rb, x, y, n, k, m, add, s);
+    if (m > 1 && (type == T_Q4_0 || type == T_Q5_0 || type == T_Q8_0)) {
+        // the prefill GEMM where its tiles fill the chip or x is long enough to be split once per tile; below
+        // that the waves of a workgroup split K (and layouts that kernel does not take run the GEMM too)
+        const bool dense = dense_ok(type, w, nullptr, rb, x, k);
+        if (!dense || gemm_us(n, k, m, false) < dense_us(n, k, m, false))
+            return gemm_f32(type, w, nullptr, rb, x, y, n, k, m, add, s);
+    }
+    if (m >= kF32GemmMinRows && f32_gemm_ok(type, w, rb, x, k) &&
+        (type != T_Q6_K || !dense_ok(type, w, nullptr, rb, x, k) || f32_gemm_us_q6k(n, k, m) <= dense_us(n, k, m, false)))
+        return f32_gemm(type, w, rb, x, y, n, k, m, add, s);
     if (m > 1 && dense_ok(type, w, nullptr, rb, x, k)) return dense_matmul(type, w, nullptr, rb, x, y, n, k, m, add, s);
     return gemv_generic(type, w, rb, x, y, n, k, m, add, s);
 }

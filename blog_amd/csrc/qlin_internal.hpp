@@ -133,16 +133,29 @@ hipError_t dequant(int type, const uint8_t *src, void *out, int64_t n, bool to_f
 
 // Q8_1 activation quantizer (36 B per 32 values) and the weight x Q8_1 matmul.
 hipError_t quantize_q8_1(const float *x, uint8_t *xq, int in_dim, int m, bool raw_sum, hipStream_t s);
+// The prefill GEMM of the 32-block formats (Q4_0, Q5_0, Q8_0) on the fp16 matrix cores (qlin_gemm.hip): f32
+// activations (mode 0: y =, 1: y +=, 2: SwiGLU of the gate rows w0 and the up rows w1) or Q8_1 ones, any
+// layout the entry points accept.  gemm_us, dense_us: the estimated microseconds of gemm_f32 and of
+// dense_matmul (all formats but Q4_K), from which the dispatch chooses.
+float gemm_us(int n, int k, int m, bool swiglu);
+float dense_us(int n, int k, int m, bool swiglu);
+hipError_t gemm_f32(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, float *y, int n,
+                    int k, int m, int mode, hipStream_t s);
+hipError_t gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, float *y, int n, int k, int m,
+                     hipStream_t s);
 // Q8_0 / Q5_0 / Q4_0 x Q8_1 prefill GEMM on the fp16 matrix cores (qlin_qblk_gemm.hip).
 bool qblk_gemm_ok(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, int in_dim);
+float qblk_gemm_us(int out_dim, int in_dim, int m);  // its estimated microseconds (not Q6_K's)
 hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, float *y, int out_dim,
                           int in_dim, int m, hipStream_t s);
 // Q4_K / Q6_K x f32 activations, the prefill GEMM of quant_matmul for m >= kF32GemmMinRows rows, on the
-// fp16 matrix cores (qlin_f32_gemm.hip); fewer rows take dense_matmul.  add: y += the product.
+// fp16 matrix cores (qlin_f32_gemm.hip); fewer rows (Q6_K: also
+// products of few tiles) take dense_matmul.  add: y += the product.
 #ifndef QLIN_F32_GEMM_MIN_ROWS
 #define QLIN_F32_GEMM_MIN_ROWS 64
 #endif
 constexpr int kF32GemmMinRows = QLIN_F32_GEMM_MIN_ROWS;
+float f32_gemm_us_q6k(int out_dim, int in_dim, int m);  // its estimated microseconds for Q6_K
 bool f32_gemm_ok(int type, const uint8_t *w, size_t row_bytes, const float *x, int in_dim);
 hipError_t f32_gemm(int type, const uint8_t *w, size_t row_bytes, const float *x, float *y, int out_dim, int in_dim,
                     int m, bool add, hipStream_t s);

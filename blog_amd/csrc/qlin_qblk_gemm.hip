@@ -614,6 +614,21 @@ bool qblk_gemm_ok(int type, const uint8_t *w, size_t rb, const uint8_t *xq, int 
            (reinterpret_cast<uintptr_t>(xq) & 3u) == 0;
 }
 
+// Measured: a round of workgroups takes about 9.8 us per unit of 256 values on the default tiles, 4.7 on
+// the small ones (the 32-block formats').
+static bool small_tiles(int out_dim, int m) {
+    const int64_t large = static_cast<int64_t>((out_dim + GeoLarge::kBN - 1) / GeoLarge::kBN) *
+                          ((m + GeoLarge::kBM - 1) / GeoLarge::kBM);
+    return QLIN_QBLK_SMALL && large * 2 < device_info().cu_count;
+}
+float qblk_gemm_us(int out_dim, int in_dim, int m) {
+    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+    const bool small = small_tiles(out_dim, m);
+    const int bn = small ? GeoSmall::kBN : GeoLarge::kBN, bm = small ? GeoSmall::kBM : GeoLarge::kBM;
+    const int64_t wgs = static_cast<int64_t>((out_dim + bn - 1) / bn) * ((m + bm - 1) / bm);
+    return 3.0f + static_cast<float>((wgs + cus - 1) / cus) * (small ? 4.7f : 9.8f) * static_cast<float>((in_dim + 255) / 256);
+}
+
 hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t rb, const uint8_t *xq, float *y, int out_dim,
                           int in_dim, int m, hipStream_t s) {
     if (out_dim == 0 || m == 0) return hipSuccess;
@@ -647,9 +662,7 @@ hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t rb, const uint8_t *
     // the default: its lm_head shapes fill the chip many times).  DeepSeek-V2-Lite's Q5_0 expert down at
     // 512 tokens (64 default workgroups): 40.5 -> 23.7 us.  A Q8_0 [4864, 896] at 512 tokens (152 default
     // workgroups) ran 34.2 us on the default tiles and 45.5 us on the small ones.
-    const int64_t large = static_cast<int64_t>((out_dim + GeoLarge::kBN - 1) / GeoLarge::kBN) *
-                          ((m + GeoLarge::kBM - 1) / GeoLarge::kBM);
-    if (QLIN_QBLK_SMALL && type != T_Q6_K && large * 2 < device_info().cu_count) return launch(GeoSmall{});
+    if (type != T_Q6_K && small_tiles(out_dim, m)) return launch(GeoSmall{});
     return launch(GeoLarge{});
 }
 

@@ -515,6 +515,102 @@ def test_f32_gemm_add(qtype, m):
     assert normwise_rel_err(host(yd), ref) <= FP32
 
 
+BLOCK_ROWS = [  # (type, N, K, m): few rows and short K (a unit of blocks cut short), every tile kind, odd block counts
+    (Q8_0, 100, 96, 2), (Q5_0, 33, 1056, 17), (Q4_0, 520, 160, 40), (Q8_0, 1718, 1280, 25), (Q4_0, 4000, 544, 70),
+    (Q6_K, 70, 256, 5), (Q6_K, 300, 1280, 33), (Q6_K, 1030, 768, 130),
+    (Q8_0, 8300, 224, 130),      # the GEMM's 64 x 128 tiles, 7 blocks
+    (Q5_0, 14400, 2080, 260),    # its 128 x 256 tiles, 65 blocks
+    (Q4_0, 14400, 2048, 300)]
+
+
+@pytest.mark.parametrize("mode", ["store", "add", "swiglu"])
+@pytest.mark.parametrize("qtype,N,K,m", BLOCK_ROWS)
+def test_rows_of_f32(qtype, N, K, m, mode):
+    """Several rows of f32 activations through the split-fp16 kernels (quant_matmul, its add form, the SwiGLU
+    rows): against the f64 oracle, each output within 2e-5 of its own sum |w||x| (the bound of the other
+    f32 paths) and normwise 1e-5."""
+    w, rb, vals = qgen.random_matrix(qtype, N, K, seed=K + m)
+    x = qgen.random_x(m, K, seed=N + m)
+    banner(f"rows type={qtype} {m}x{K}x{N} {mode}")
+    toks = np.unique(np.r_[0, 15 % m, 16 % m, m // 2, m - 1])
+    xd, wd = dev(x), dev(w)
+    ref = orc.matmul_f64(qtype, w, rb, x[toks], N, K)
+    if mode == "swiglu":
+        w2, _, _ = qgen.random_matrix(qtype, N, K, seed=K + m + 1)
+        yd = empty_f32(m, N)
+        qlin.quant_swiglu_rows(qtype, wd, dev(w2), rb, rb, xd, yd, N, K, m)
+        u = orc.matmul_f64(qtype, w2, rb, x[toks], N, K)
+        with np.errstate(over="ignore"):
+            ref = ref / (1.0 + np.exp(-ref)) * u
+        got = host(yd)
+        assert np.isfinite(got).all()
+        assert normwise_rel_err(got[toks], ref) <= 2 * FP32   # a product of two such sums
+        return
+    y0 = np.random.default_rng(5).standard_normal((m, N)).astype(np.float32)
+    yd = dev(y0) if mode == "add" else empty_f32(m, N)
+    (qlin.quant_matmul_add if mode == "add" else qlin.quant_matmul)(qtype, wd, rb, xd, yd, N, K, m)
+    got = host(yd)
+    assert np.isfinite(got).all()
+    if mode == "add":
+        ref = ref + y0[toks]
+    scale = np.abs(x[toks].astype(np.float64)) @ np.abs(vals.astype(np.float64)).T + 1.0
+    assert np.max(np.abs(got[toks] - ref) / scale) <= COND
+    assert normwise_rel_err(got[toks], ref) <= FP32
+
+
+@pytest.mark.parametrize("qtype,N,m", [(Q8_0, 300, 70), (Q6_K, 300, 40), (Q4_0, 8300, 130)])
+def test_rows_of_f32_token_scales(qtype, N, m):
+    """Tokens of very different magnitudes, one whose large values come last or first (the scale changes on
+    the way), zeros, and an infinite or NaN value, which reaches its own token's outputs alone."""
+    K = 1024
+    w, rb, vals = qgen.random_matrix(qtype, N, K, seed=195)
+    rng = np.random.default_rng(196)
+    x = rng.standard_normal((m, K)).astype(np.float32)
+    mags = [1e-30, 1e-12, 1e-3, 1.0, 1e3, 1e12, 1e30]
+    for i in range(m):
+        x[i] *= np.float32(mags[i % len(mags)])
+    x[10] = 0.0
+    x[11] = np.float32(1e-6) * rng.standard_normal(K)
+    x[11, 1000] = 1e6
+    x[12] = rng.standard_normal(K) * np.logspace(-20, 20, K)
+    x[13] = rng.standard_normal(K) * np.logspace(20, -20, K)
+    x[14, :512] = 0.0
+    x[15, 77], x[16, 900], x[17, 500] = np.inf, -np.inf, np.nan
+    banner(f"rows token scales type={qtype} N={N}")
+    yd = empty_f32(m, N)
+    qlin.quant_matmul(qtype, dev(w), rb, dev(x), yd, N, K, m)
+    got = host(yd)
+    fine = np.r_[0:15, 18:m]
+    ref = orc.matmul_f64(qtype, w, rb, x[fine], N, K)
+    scale = np.abs(x[fine].astype(np.float64)) @ np.abs(vals.astype(np.float64)).T
+    err = np.abs(got[fine] - ref) / np.maximum(scale.max(axis=1, keepdims=True), 1e-300)
+    assert np.isfinite(got[fine]).all() and err.max() <= COND, float(err.max())
+    assert not got[10].any()
+    for t, k in ((15, 77), (16, 900)):           # w inf: infinite with the weight's sign, NaN for a zero weight
+        wk = vals[:, k].astype(np.float64)
+        assert np.isnan(got[t][wk == 0]).all()
+        assert (got[t][wk != 0] == np.sign(wk[wk != 0]) * x[t, k]).all()
+    assert np.isnan(got[17]).all()
+
+
+@pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 14400, 1088, 257), (Q5_0, 14400, 1024, 130), (Q4_0, 70, 96, 5),
+                                         (Q8_0, 300, 1056, 66)])
+def test_matmul_q8_1_shared_gemm(qtype, N, K, m):
+    """Q8_1 activations through the GEMM shared with f32 ones: full tiles, and odd block counts, which the
+    64-token kernel does not take; against the oracle's block dots."""
+    w, rb, _ = qgen.random_matrix(qtype, N, K, seed=K + N)
+    x = qgen.random_x(m, K, seed=m)
+    xq = orc.quantize_q8_1(x.reshape(-1), m * K)
+    banner(f"q8_1 shared gemm type={qtype} {m}x{K}x{N}")
+    yd = empty_f32(m, N)
+    qlin.quant_matmul_q8_1(qtype, dev(w), rb, dev(xq), yd, N, K, m)
+    toks = np.unique(np.r_[0, m // 2, m - 1])
+    rbx = orc.q8_1_row_bytes(K)
+    ref = orc.matmul_q8_1(qtype, w, rb, np.ascontiguousarray(xq.reshape(m, rbx)[toks]).reshape(-1), N, K, toks.size)
+    assert np.isfinite(host(yd)).all()
+    assert normwise_rel_err(host(yd)[toks], ref) <= FP32
+
+
 # ---- MoE ----------------------------------------------------------------------------------------
 
 # up to 64 experts take the one-pass rank kernel, more the k-round argmax kernel
