@@ -88,6 +88,25 @@ def _same_bits(got, ref, what):
                     f"expected {ref[i].tolist()}")
 
 
+@pytest.mark.parametrize("qtype", [Q4_0, Q5_0, Q8_0, Q4_K, Q6_K])
+@pytest.mark.parametrize("nb", [1, 67])
+def test_dequant_few_blocks_offset(qtype, nb):
+    """One block and a count that leaves the last workgroup short, source and output one element off their
+    vectors' alignment: every value, and nothing around them."""
+    w, _ = qgen.random_blocks(qtype, nb, np.random.default_rng(qtype + nb))
+    n = nb * qgen.BLOCK[qtype][0]
+    banner(f"dequant offset type={qtype} blocks={nb}")
+    wd = dev(np.concatenate([np.zeros(2, np.uint8), w]))[2:]
+    o16 = torch.full((n + 2,), 77, dtype=torch.int16, device="cuda")
+    o32 = torch.full((n + 2,), 77.0, dtype=torch.float32, device="cuda")
+    qlin.dequantize(qtype, wd, o16[1:], n, f16=True)
+    qlin.dequantize(qtype, wd, o32[1:], n, f16=False)
+    h16, h32 = host(o16), host(o32)
+    _same_bits(h32[1:-1].view(np.uint32), orc.dequant_f32(qtype, w, n).view(np.uint32), "f32")
+    _same_bits(h16[1:-1].view(np.uint16), orc.dequant_f16(qtype, w, n), "f16")
+    assert h16[0] == h16[-1] == 77 and h32[0] == h32[-1] == 77.0
+
+
 def test_dequant_reference_names():
     w = qgen.random_matrix(Q4_K, 4, 512, seed=3)[0]
     n = 4 * 512
