@@ -240,6 +240,168 @@ __global__ __launch_bounds__(kAttnThreads) void attend_kernel(const float *__res
     }
 }
 
+// Several rows (a prompt): a workgroup per (16 rows, query head), its 8 waves taking 16 positions at a time in
+// turn, on v_mfma_f32_16x16x4_f32 (f32 operands and sums, as above).  Scores: lane (n, g) holds dims
+// DG g .. of query row n and of position n's key (DG = HD / 4), so MFMA i multiplies dims DG g + i in k-slot
+// g.  Each wave keeps its rows' running maximum, sum and output (rescaled when the maximum grows), turns its
+// probabilities into the A layout in LDS, and multiplies value rows 4g + i in k-slot g; the waves' outputs
+// meet in LDS.  Positions past a row's own score -inf.  Four score chains and an output sum per tile keep the
+// error against float64 at or below attend_kernel's (at 30000 positions 4.5e-7 against 1.0e-6; one chain each
+// had 2.0e-6).  Bound by the latency of a wave's few tiles.  attend_kernel reads every key and value row again
+// for each query row: 384 rows of 14 heads of 64 from position 0 54 us, here 16; 2000 rows 1195 us, here 147;
+// 512 rows of 32 heads of 128 368 us, here 90.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true)));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+// over the 16 lanes of a row
+__device__ __forceinline__ float max_of_16(float v) { return dpp_max<0x140>(dpp_max<0x141>(dpp_max<0x4e>(dpp_max<0xb1>(v)))); }
+__device__ __forceinline__ float sum_of_16(float v) { return dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4e>(dpp_add<0xb1>(v)))); }
+
+constexpr int kRowWaves = 8;
+template <int HD>
+__global__ __launch_bounds__(64 * kRowWaves) void attend_rows_kernel(const float *__restrict__ q,
+                                                                     const float *__restrict__ kc,
+                                                                     const float *__restrict__ vc, float *__restrict__ out,
+                                                                     int rows, int n_heads, int kv_heads, int max_seq,
+                                                                     const int *__restrict__ start_pos) {
+    constexpr int DG = HD / 4, CT = HD / 16;
+    __shared__ f32x4 s_p[kRowWaves][16][5];  // (rows of 20 floats: 16 probabilities)
+    __shared__ float s_o[kRowWaves][16][HD], s_m[kRowWaves][16], s_l[kRowWaves][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+    const int r0 = blockIdx.x * 16, h = blockIdx.y, kh = h / (n_heads / kv_heads);
+    const int start = *start_pos;
+    auto pos_of = [&](int row) { return min(max(start + row, 0), max_seq - 1); };
+    const int last = pos_of(min(r0 + 15, rows - 1));  // rows' positions never fall
+    const int first = pos_of(r0);
+    const size_t stride = static_cast<size_t>(kv_heads) * HD;
+    const float *kb = kc + static_cast<size_t>(kh) * HD, *vb = vc + static_cast<size_t>(kh) * HD;
+    const float scale = rsqrtf(static_cast<float>(HD));
+
+    f32x4 qv[DG / 4];
+    {
+        const f32x4 *p = reinterpret_cast<const f32x4 *>(q + (static_cast<size_t>(min(r0 + n, rows - 1)) * n_heads + h) * HD + DG * g);
+#pragma unroll
+        for (int i = 0; i < DG / 4; ++i) qv[i] = p[i];
+    }
+    int pr[4];
+    float m[4], l[4];
+    f32x4 O[CT];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        pr[r] = pos_of(min(r0 + 4 * g + r, rows - 1));
+        m[r] = -INFINITY;
+        l[r] = 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < CT; ++c) O[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    f32x4 kv[DG / 4];
+    float vv[4][CT];
+    auto load = [&](int t0) {  // past the last position: that one again (its probabilities are 0)
+        const f32x4 *p = reinterpret_cast<const f32x4 *>(kb + static_cast<size_t>(min(t0 + n, last)) * stride + DG * g);
+#pragma unroll
+        for (int i = 0; i < DG / 4; ++i) kv[i] = p[i];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) vv[i][c] = vb[static_cast<size_t>(min(t0 + 4 * g + i, last)) * stride + 16 * c + n];
+    };
+    int t0 = 16 * wave;
+    if (t0 <= last) load(t0);
+    for (; t0 <= last; t0 += 16 * kRowWaves) {  // uniform
+        f32x4 S4[4] = {};  // four chains: a quarter of the latency, and of the rounding
+#pragma unroll
+        for (int i = 0; i < DG; ++i)
+            S4[i % 4] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[i / 4][i % 4], kv[i / 4][i % 4], S4[i % 4], 0, 0, 0);
+        f32x4 S;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[r] = (S4[0][r] + S4[1][r]) + (S4[2][r] + S4[3][r]);
+        float al[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float s = t0 + n <= pr[r] ? S[r] * scale : -INFINITY;
+            const float mn = fmaxf(m[r], max_of_16(s)), mu = mn == -INFINITY ? 0.0f : mn;
+            al[r] = expf(m[r] - mu);
+            const float p = expf(s - mu);
+            m[r] = mn;
+            l[r] = l[r] * al[r] + p;
+            reinterpret_cast<float *>(s_p[wave][4 * g + r])[n] = p;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the wave's own rows of s_p)
+        __builtin_amdgcn_wave_barrier();
+        const f32x4 pa = s_p[wave][n][g];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) O[c][r] *= al[r];
+        bool odd = false;  // a value that is not finite at a position that some row does not see
+        if (t0 + 15 > first) {  // uniform
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) odd |= !isfinite(vv[i][c]);
+        }
+        if (__any(odd)) {  // uniform: 0 times that value would be NaN
+            for (int j = 0; j < 16 && t0 + j <= last; ++j) {
+                const float *vj = vb + static_cast<size_t>(t0 + j) * stride + n;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (t0 + j > pr[r]) continue;
+                    const float p = reinterpret_cast<const float *>(s_p[wave][4 * g + r])[j];
+#pragma unroll
+                    for (int c = 0; c < CT; ++c) O[c][r] = fmaf(p, vj[16 * c], O[c][r]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {  // the tile's own sum, then added: a shorter chain of roundings
+                f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[i], vv[i][c], t, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) O[c][r] += t[r];
+            }
+        }
+        if (t0 + 16 * kRowWaves <= last) load(t0 + 16 * kRowWaves);  // uniform
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        l[r] = sum_of_16(l[r]);
+        if (n == 0) {
+            s_m[wave][4 * g + r] = m[r];
+            s_l[wave][4 * g + r] = l[r];
+        }
+#pragma unroll
+        for (int c = 0; c < CT; ++c) s_o[wave][4 * g + r][16 * c + n] = O[c][r];
+    }
+    __syncthreads();
+    for (int e = tid; e < 16 * HD; e += 64 * kRowWaves) {
+        const int row = e / HD, d = e % HD;
+        if (r0 + row >= rows) continue;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kRowWaves; ++w) mx = fmaxf(mx, s_m[w][row]);
+        float num = 0.0f, den = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kRowWaves; ++w) {
+            const float mw = s_m[w][row], lw = s_l[w][row];
+            if (mw == -INFINITY && lw == 0.0f) continue;  // no position of this row
+            const float f = mw == -INFINITY ? 1.0f : expf(mw - mx);  // (then lw is NaN)
+            num = fmaf(s_o[w][row][d], f, num);
+            den = fmaf(lw, f, den);
+        }
+        out[(static_cast<size_t>(r0 + row) * n_heads + h) * HD + d] = num / den;
+    }
+}
+
 hipStream_t current_stream() { return static_cast<hipStream_t>(qlin_get_stream()); }
 int launched(hipError_t e) { return e == hipSuccess ? QLIN_OK : QLIN_ERR_LAUNCH; }
 bool al4(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
@@ -291,6 +453,20 @@ int qlin_launch_attend(const float *q, const float *key_cache, const float *valu
     if (!qlin::al16(q) || !qlin::al16(key_cache) || !qlin::al16(value_cache) || !qlin::al16(attn) ||
         !qlin::al4(start_pos_dev))
         return QLIN_ERR_ALIGN;
+    // Whole groups of 16 rows, and enough (row, head) pairs that attend_kernel's workgroups would wait for one
+    // another: the position is not known here, and from 448 pairs on attend_rows_kernel is the faster one from
+    // the cache's start to its end (32 rows of 14 heads at 0: 6.0 -> 5.2 us, at 1500: 39.2 -> 29.8; 16 rows of
+    // 32 heads of 128 at 3000: 146 -> 111), while 16 rows of 14 heads at 1500 take 26.9 us there and 29.6 here.
+    if (rows >= 16 && static_cast<int64_t>(rows) * n_heads >= 448 && (head_dim == 64 || head_dim == 128)) {
+        const dim3 grid((rows + 15) / 16, n_heads), block(64 * qlin::kRowWaves);
+        if (head_dim == 64)
+            hipLaunchKernelGGL(qlin::attend_rows_kernel<64>, grid, block, 0, qlin::current_stream(), q, key_cache,
+                               value_cache, attn, rows, n_heads, kv_heads, max_seq_len, start_pos_dev);
+        else
+            hipLaunchKernelGGL(qlin::attend_rows_kernel<128>, grid, block, 0, qlin::current_stream(), q, key_cache,
+                               value_cache, attn, rows, n_heads, kv_heads, max_seq_len, start_pos_dev);
+        return qlin::launched(hipGetLastError());
+    }
     // q, then the scores of every position up to max_seq_len, later the classes' output sums (at most
     // 256 threads' float4s), in LDS
     const size_t slots = static_cast<size_t>(qlin::kAttnThreads) * 4;

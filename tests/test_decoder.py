@@ -355,6 +355,50 @@ def test_rms_norm_fused_unsupported_shape():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,nh,nkv,d,s,start", [(32, 14, 2, 64, 512, 250), (33, 28, 4, 128, 512, 0), (17, 32, 8, 128, 160, 127),
+                                                   (31, 15, 1, 64, 64, 50), (448, 1, 1, 128, 512, 0), (40, 16, 2, 96, 64, 3),
+                                                   (31, 14, 2, 64, 512, 250), (32, 14, 2, 64, 32, -3)])
+def test_attend_of_row_groups(rows, nh, nkv, d, s, start):
+    """Prompt attention at the edges of its groups of 16 rows, of its tiles of 16 positions and of the choice of
+    kernel, clamped positions included, against float64; values that are not finite at positions that only later
+    rows see, and past every row's, leave the earlier rows finite.  Bound: scores of magnitude <= 8 with d
+    roundings of 2^-24 each in their sums, and as many in the weighted mean: 16 d 2^-24 in norm, far above
+    what chance leaves of it."""
+    torch = _gpu()
+    from gpu_util import banner, dev, empty_f32, host
+    from blog_amd import qlin
+    rng = np.random.default_rng(rows * 1000 + d + start)
+    q = rng.standard_normal((rows, nh, d)).astype(np.float32)
+    kc, vc = (rng.standard_normal((s, nkv, d)).astype(np.float32) for _ in range(2))
+    banner(f"attend rows={rows} heads={nh}/{nkv} d={d} start={start}")
+    pos = torch.tensor([start], dtype=torch.int32, device="cuda")
+    at = [min(max(start + r, 0), s - 1) for r in range(rows)]
+
+    def run(values):
+        attn = empty_f32(rows, nh, d)
+        qlin.call("qlin_launch_attend", dev(q), dev(kc), dev(values), attn, rows, nh, nkv, d, s, pos)
+        return host(attn).reshape(rows, nh, d)
+
+    kd, vd = (np.repeat(c.astype(np.float64), nh // nkv, axis=1) for c in (kc, vc))
+    ref = np.empty((rows, nh, d))
+    for r, p in enumerate(at):
+        w = np.einsum("hd,jhd->hj", q[r].astype(np.float64), kd[:p + 1]) / np.sqrt(d)
+        w = np.exp(w - w.max(axis=1, keepdims=True))
+        ref[r] = np.einsum("hj,jhd->hd", w / w.sum(axis=1, keepdims=True), vd[:p + 1])
+    tol = 16 * d * 2.0 ** -24
+    assert normwise_rel_err(run(vc), ref) <= tol
+    bad = vc.copy()
+    bad[at[-1]] = np.inf
+    bad[at[-1], :, 0] = np.nan
+    bad[at[-1] + 1:] = np.nan
+    got = run(bad)
+    seen = np.array(at) == at[-1]
+    assert not np.isfinite(got[seen]).any()
+    if not seen.all():
+        assert normwise_rel_err(got[~seen], ref[~seen]) <= tol
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,start", [(1, 0), (1, 37), (32, 0), (5, 250), (3, 509), (1, 600)])
 def test_rope_store_and_attend(rows, start):
     """Rotary pairs, the cache store at each row's position (a position past the cache clamped to its
