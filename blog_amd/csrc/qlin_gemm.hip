@@ -53,6 +53,7 @@ template <int MT_, int NT_, int WM_, int WN_>
 struct Geo {
     static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = WN_;
     static constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN;
+    static constexpr int waves = MT * NT > 8 ? 2 : 4;  // per SIMD: two workgroups on a CU where LDS has room for them
     static_assert(WM * WN == kWaves, "8 waves");
 };
 
@@ -229,7 +230,7 @@ __device__ __forceinline__ void decode(const WRaw<FMT> &r, Put put) {
 }
 
 template <int FMT, bool Q81, int MODE, class G>
-__global__ __launch_bounds__(kThreads) void gemm_kernel(const GemmArgs a) {
+__global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs a) {
     using L = Lds<G>;
     constexpr int MT = G::MT, NT = G::NT, BM = G::BM, BN = G::BN;
     constexpr int kOut = MODE == kSwiGLU ? BN / 2 : BN;  // output columns per workgroup
@@ -524,8 +525,10 @@ using Large = Geo<4, 4, 2, 4>;  // 128 tokens x 256 rows
 using Mid = Geo<2, 2, 2, 4>;    // 64 tokens x 128 rows
 
 // Microseconds of a launch, measured: a step of a round of workgroups takes 2.5 us with the large tiles
-// (matrix cores, vector ALU and LDS each about half busy) and 1.35 us with the middle ones (a step's
-// latency), and filling and draining 12 and 6 us.
+// (matrix cores, vector ALU and LDS each about half busy); with the middle ones 1.35 us for one workgroup
+// on a CU (a step's latency) and 1.75 us for two, which LDS and registers have room for (Q8_0 [14336, 4096] at
+// 256 tokens 157 us with the large tiles, 117 with two of the middle ones; [28672, 1024] at 128 tokens 47 us
+// with one middle one after the other, 35 with two at a time).  Filling and draining: 12 and 6 us.
 struct GemmPlan {
     bool large;
     float us;
@@ -533,13 +536,14 @@ struct GemmPlan {
 GemmPlan gemm_plan(int n, int k, int m, bool swiglu) {
     const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
     const float steps = static_cast<float>((k / 32 + 1) / 2);
-    auto rounds = [&](int bm, int bn) {
+    auto groups = [&](int bm, int bn) {
         if (swiglu) bn /= 2;
-        const int64_t wgs = static_cast<int64_t>((n + bn - 1) / bn) * ((m + bm - 1) / bm);
-        return static_cast<float>((wgs + cus - 1) / cus);
+        return static_cast<int64_t>((n + bn - 1) / bn) * ((m + bm - 1) / bm);
     };
-    const float l = 12.0f + 2.5f * steps * rounds(Large::BM, Large::BN);
-    const float d = 6.0f + 1.35f * steps * rounds(Mid::BM, Mid::BN);
+    const int64_t lg = groups(Large::BM, Large::BN), mg = groups(Mid::BM, Mid::BN), rest = mg % (2 * cus);
+    const float l = 12.0f + 2.5f * steps * static_cast<float>((lg + cus - 1) / cus);
+    const float d = 6.0f + steps * (1.75f * static_cast<float>(mg / (2 * cus)) +
+                                    (rest == 0 ? 0.0f : rest <= cus ? 1.35f : 1.75f));
     return l <= d ? GemmPlan{true, l} : GemmPlan{false, d};
 }
 
