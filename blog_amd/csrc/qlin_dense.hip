@@ -528,10 +528,8 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
         };
         tile(0);
         if constexpr (TT > 1) tile(1);
-        if constexpr (TT > 2) {
-            tile(2);
-            tile(3);
-        }
+        if constexpr (TT > 2) tile(2);
+        if constexpr (TT > 3) tile(3);
     }
     __syncthreads();  // (the sums below take the LDS of the tiles)
 
@@ -575,8 +573,9 @@ hipError_t launch_rows(const DenseArgs &a, hipStream_t s) {
 
 // The tiles of a launch: NT row tiles (of a SwiGLU: NT / 2 outputs') by TT token tiles per workgroup, one
 // workgroup on a CU at a time.  Measured, a round of workgroups takes about 2 us plus, per unit of a wave,
-// 2.1 (1 x 1), 3.3 (2 x 1), 3.2 (1 x 2), 4.6 (2 x 2) and 8.8 us (2 x 4): larger tiles split x and read the
-// weights for more products, smaller ones fill the chip.  The cheapest total is taken.
+// 2.1 (1 x 1), 3.3 (2 x 1), 3.2 (1 x 2), 4.6 (2 x 2), 6.6 (2 x 3) and 8.8 us (2 x 4): larger tiles split x and read the
+// weights for more products, smaller ones fill the chip.  The cheapest total is taken (Q8_0 [896, 4864] at 384
+// tokens: 168 workgroups of 2 x 4 tiles 44 us, 224 of 2 x 3 32 us).
 struct RowsPlan {
     int nt, tt;
     float us;
@@ -585,7 +584,7 @@ RowsPlan rows_plan(int n, int k, int m, bool swiglu) {
     static constexpr struct {
         int nt, tt;
         float unit;
-    } kinds[] = {{1, 1, 2.1f}, {2, 1, 3.3f}, {1, 2, 3.2f}, {2, 2, 4.6f}, {2, 4, 8.8f}};
+    } kinds[] = {{1, 1, 2.1f}, {2, 1, 3.3f}, {1, 2, 3.2f}, {2, 2, 4.6f}, {2, 3, 6.6f}, {2, 4, 8.8f}};
     const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
     const float units = static_cast<float>((k / 32 + kUnit * kDWaves - 1) / (kUnit * kDWaves));
     RowsPlan best{0, 0, 0.0f};
@@ -608,6 +607,7 @@ hipError_t by_shape(const DenseArgs &a, hipStream_t s) {
     switch (p.tt) {
         case 1: return launch_rows<T, MODE, 2, 1>(a, s);
         case 2: return launch_rows<T, MODE, 2, 2>(a, s);
+        case 3: return launch_rows<T, MODE, 2, 3>(a, s);
         default: return launch_rows<T, MODE, 2, 4>(a, s);
     }
 }

@@ -539,7 +539,9 @@ BLOCK_ROWS = [  # (type, N, K, m): few rows and short K (a unit of blocks cut sh
     (Q6_K, 70, 256, 5), (Q6_K, 300, 1280, 33), (Q6_K, 1030, 768, 130),
     (Q8_0, 8300, 224, 130),      # the GEMM's 64 x 128 tiles, 7 blocks
     (Q5_0, 14400, 2080, 260),    # its 128 x 256 tiles, 65 blocks
-    (Q4_0, 14400, 2048, 300)]
+    (Q4_0, 14400, 2048, 300),
+    (Q8_0, 8300, 224, 270),      # two workgroups on a CU
+    (Q8_0, 890, 160, 370), (Q5_0, 890, 1056, 370), (Q4_0, 890, 160, 370), (Q6_K, 900, 256, 380)]  # 2 x 3 tiles
 
 
 @pytest.mark.parametrize("mode", ["store", "add", "swiglu"])
