@@ -17,11 +17,12 @@
 // 4g+3 of row l % 16.  The waves' partials meet in LDS and are summed in wave order.  A grid row per 64
 // tokens.
 #include "qlin_device.hpp"
+#include "qlin_bf16x3.hpp"
 #include "qlin_internal.hpp"
 #include "qlin_mfma.hpp"
+#include "qlin_plan.hpp"
 #include "qlin_rows.hpp"
 #include "qlin_values8.hpp"
-#include <type_traits>
 
 namespace qlin {
 namespace {
@@ -172,38 +173,20 @@ __global__ __launch_bounds__(kDThreads) void q4k_dense_kernel(const DenseArgs a)
 
 // ---- the other formats (Q4_0, Q5_0, Q8_0, Q6_K) --------------------------------------------------
 //
-// v_mfma_f32_16x16x32_f16 with the tokens as the MFMA rows, the operands of the prefill GEMM
-// (qlin_gemm.hip): B = q less its offset (Q6_K: sc (q - 32) in two exact parts), A = x 2^s split into fp16
-// hi and lo, s per token from its largest magnitude so far (rescaled when a value 8 times that comes).
+// The tokens are the MFMA rows; x enters in its three exact bf16 parts and the weights as integers
+// (qlin_bf16x3.hpp).  32-block formats: v_mfma_f32_16x16x32_bf16, one scale per block.  Q6_K, whose scales
+// are per 16 values: v_mfma_f32_16x16x16_bf16, one scale d sc (exact in f32) per MFMA sum.
 // Nothing is shared between waves: each takes whole units of four 32-blocks of K in turn (wave w: w, w + 8,
 // ...) for all of the workgroup's rows and tokens, straight from memory, one unit's weights and one token
 // tile's x ahead, so short and narrow products need no barrier per step; the waves' sums meet in LDS.
-// What bounds it: a tile's chain (x turned in LDS, its scale, 64 split and 16-32 scaling instructions
-// around 8-16 MFMAs) with two waves on a SIMD.  A request whose lanes lie in different rows costs the
-// address path a cycle per lane, which is why x is read along its rows and a lane group reads a whole
-// block.  Against f32 matrix cores (v_mfma_f32_16x16x4_f32) on decoded values with the layout's own
-// 8-byte pieces: Q6_K [3584, 18944] at 12 rows 78 -> 33 us, Q5_0 [4096, 4096] at 6 rows 19 -> 10 us, Q8_0
-// [4096, 4096] at 100 rows 108 -> 38 us, Q5_0 [30000, 1024] at 40 rows 92 -> 26 us.
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ f32x4 mfma_h(const uint4 &a, const uint4 &b, const f32x4 &c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ uint32_t h2u(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
-__device__ __forceinline__ f16x2 u2h(uint32_t u) { return __builtin_bit_cast(f16x2, u); }
-__device__ __forceinline__ f16x2 splat(float v) {
-    const _Float16 h = static_cast<_Float16>(v);
-    return f16x2{h, h};
-}
-// the fp16 pairs 1024 + byte of bytes 0, 1 and 2, 3
-__device__ __forceinline__ f16x2 bytes_lo(uint32_t v) { return u2h(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)); }
-__device__ __forceinline__ f16x2 bytes_hi(uint32_t v) { return u2h(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)); }
-__device__ __forceinline__ uint4 minus8(uint32_t a, uint32_t b, f16x2 off) {
-    return make_uint4(h2u(bytes_lo(a) + off), h2u(bytes_hi(a) + off), h2u(bytes_lo(b) + off), h2u(bytes_hi(b) + off));
-}
-__device__ __forceinline__ uint32_t bit4_of_bytes(uint32_t b) { return (__umul24(b & 0xfu, 0x204081u) & 0x01010101u) << 4; }
+// A request whose lanes lie in different rows costs the address path a cycle per lane, which is why x is read
+// along its rows and a lane group reads a whole block.
+// What bounds it: a tile's chain (x turned in LDS, 176 instructions to split its 32 values a lane, 12-24 MFMAs and
+// their scaling) with two or three waves on a SIMD.  Against f32 matrix cores (v_mfma_f32_16x16x4_f32) on decoded
+// values: Q6_K [3584, 18944] at 12 rows 78 -> 33 us, Q5_0 [4096, 4096] at 6 rows 18.4 -> 9.2 us, Q8_0 [4096, 4096]
+// at 100 rows 107 -> 32 us; 2-norm error against f64 over N(0, 1) x of 2048 values 2.9e-7 -> 0.9e-7 (1.0e-7 as an
+// fp16 pair under a scale per token, at the same times).  149 registers (1 x 1) to 256 (2 x 4: 0 to 6 of them
+// spilled, Q6_K's 2 x 3 up to 2; the measured costs in qlin_plan.hpp include them).
 
 constexpr int kUnit = 4;  // 32-blocks of a unit
 
@@ -237,6 +220,7 @@ __device__ __forceinline__ void all_groups(uint32_t v, uint32_t (&o)[4]) {
 template <int T>
 struct Unit {
     static constexpr int W = T == T_Q8_0 ? 8 : 4;
+    static constexpr int kScales = kUnit;  // the unit's scales
     uint32_t q[W], d, qh;
     __device__ __forceinline__ void load(const uint8_t *row, int blk, int last, int g) {
         const uint8_t *b = row + static_cast<size_t>(min(blk + g, last)) * Block<T>::bytes;
@@ -252,7 +236,7 @@ struct Unit {
         }
     }
     // the operands and scales of the unit's blocks
-    __device__ __forceinline__ void operands(int g, uint4 (&b)[kUnit], uint4 (&)[1], float (&dw)[kUnit]) const {
+    __device__ __forceinline__ void operands(int g, u32x4 (&b)[kUnit], float (&dw)[kScales]) const {
         uint32_t ds[4], o[kUnit][2];
         all_groups(d, ds);
 #pragma unroll
@@ -285,7 +269,7 @@ struct Unit {
         for (int j = 0; j < kUnit; ++j) {
             dw[j] = f16_bits_to_f32(ds[j]);
             if constexpr (T == T_Q8_0) {
-                b[j] = minus8(o[j][0] ^ 0x80808080u, o[j][1] ^ 0x80808080u, splat(-1152.0f));
+                b[j] = bf16_of_i8(o[j][0], o[j][1]);
             } else {  // low nibbles: elements 0..15, high: 16..31
                 uint32_t u = (o[j][0] >> (4 * (g >> 1))) & 0x0f0f0f0fu, v = (o[j][1] >> (4 * (g >> 1))) & 0x0f0f0f0fu;
                 if constexpr (T == T_Q5_0) {
@@ -293,13 +277,19 @@ struct Unit {
                     u |= bit4_of_bytes(hb);
                     v |= bit4_of_bytes(hb >> 4);
                 }
-                b[j] = minus8(u, v, splat(T == T_Q5_0 ? -1040.0f : -1032.0f));
+                b[j] = bf16_of_u8(u, v, T == T_Q5_0 ? 16.0f : 8.0f);
             }
         }
     }
+    // x's slot (f32x4) e of the unit for lane group g: elements 8g + 4 (e & 1) .. + 3 of block e / 2
+    static __device__ __forceinline__ int x_slot(int e, int g) { return 8 * (e >> 1) + 2 * g + (e & 1); }
 };
+// Half a super-block.  A lane reads bytes 8g .. 8g+7 of each 32, of one 16-value group for lanes of groups 0
+// and 1, of the other for 2 and 3; after the swap every lane has 4 values of each 16-group: group g of
+// 16-group s has its elements 8 (g & 1) + 4 (g >> 1) .. + 3.  b[j]: those of 16-groups 2j and 2j + 1.
 template <>
-struct Unit<T_Q6_K> {  // half a super-block
+struct Unit<T_Q6_K> {
+    static constexpr int kScales = 2 * kUnit;
     uint2 l[2], h, sc;
     uint32_t d;
     __device__ __forceinline__ void load(const uint8_t *row, int blk, int, int g) {
@@ -311,67 +301,30 @@ struct Unit<T_Q6_K> {  // half a super-block
         sc = ld8_a2(sb + 192 + 8 * half);
         d = ld_u16(sb + 208);
     }
-    __device__ __forceinline__ void operands(int g, uint4 (&b1)[kUnit], uint4 (&b2)[kUnit], float (&dw)[kUnit]) const {
-        dw[0] = f16_bits_to_f32(d);
+    __device__ __forceinline__ void operands(int, u32x4 (&b)[kUnit], float (&dw)[kScales]) const {
+        const float df = f16_bits_to_f32(d);
+        uint2 lo[2] = {l[0], l[1]}, hi = h;
+        swap32(lo[0].x, lo[0].y);
+        swap32(lo[1].x, lo[1].y);
+        swap32(hi.x, hi.y);
 #pragma unroll
-        for (int j = 0; j < kUnit; ++j) operand(j, g, b1[j], b2[j]);
-    }
-    __device__ __forceinline__ void operand(int j, int g, uint4 &b1, uint4 &b2) const {
-        const uint32_t s = (((j < 2 ? sc.x : sc.y) >> (8 * (2 * (j & 1) + (g >> 1)))) & 0xffu) ^ 0x80u;
-        const f16x2 s2 = u2h(0x64006400u | s | (s << 16)) + splat(-1152.0f);
-        const uint2 lw = l[j & 1];
-        const uint32_t u = ((lw.x >> (4 * (j >> 1))) & 0x0f0f0f0fu) | (((h.x >> (2 * j)) & 0x03030303u) << 4);
-        const uint32_t v = ((lw.y >> (4 * (j >> 1))) & 0x0f0f0f0fu) | (((h.y >> (2 * j)) & 0x03030303u) << 4);
-        const uint4 q = minus8(u, v, splat(-1056.0f));
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-        uint32_t p1[4], p2[4];
+        for (int j = 0; j < kUnit; ++j) {
+            const uint2 lw = lo[j & 1];
+            const uint32_t u = ((lw.x >> (4 * (j >> 1))) & 0x0f0f0f0fu) | (((hi.x >> (2 * j)) & 0x03030303u) << 4);
+            const uint32_t v = ((lw.y >> (4 * (j >> 1))) & 0x0f0f0f0fu) | (((hi.y >> (2 * j)) & 0x03030303u) << 4);
+            b[j] = bf16_of_u8(u, v, 32.0f);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const f16x2 p = u2h(w[e]) * s2;
-            p1[e] = h2u(p);
-            p2[e] = h2u(__builtin_elementwise_fma(u2h(w[e]), s2, -p));
+            for (int s = 0; s < 2; ++s)
+                dw[2 * j + s] = mul_rn(df, static_cast<float>(static_cast<int8_t>((j < 2 ? sc.x : sc.y) >> (8 * (2 * (j & 1) + s)))));
         }
-        b1 = make_uint4(p1[0], p1[1], p1[2], p1[3]);
-        b2 = make_uint4(p2[0], p2[1], p2[2], p2[3]);
     }
+    static __device__ __forceinline__ int x_slot(int e, int g) { return 4 * e + 2 * (g & 1) + (g >> 1); }
 };
 
-// max over the four lane groups of v (>= 0, whose bits order as it does): every lane gets its token's
-__device__ __forceinline__ float max_over_groups(float v) {
-    const uint32_t b = __builtin_bit_cast(uint32_t, v);
-    const auto s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-    const uint32_t c = max(static_cast<uint32_t>(s[0]), static_cast<uint32_t>(s[1]));
-    const auto t = __builtin_amdgcn_permlane32_swap(c, c, false, false);
-    return __builtin_bit_cast(float, max(static_cast<uint32_t>(t[0]), static_cast<uint32_t>(t[1])));
-}
-__device__ __forceinline__ float max3_abs(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-// hi and lo fp16 parts of 8 values times sc (a power of two)
-__device__ __forceinline__ void split8(const f32x4 &a, const f32x4 &b, float sc, uint4 &hi, uint4 &lo) {
-    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-    uint32_t h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        h[i] = h2u(f16x2{static_cast<_Float16>(fmaf(v[2 * i], sc, 0.0f)), static_cast<_Float16>(fmaf(v[2 * i + 1], sc, 0.0f))});
-        asm("" : "+v"(h[i]));  // one packed value (its halves would otherwise be formed twice)
-        const f16x2 hp = u2h(h[i]);
-        l[i] = h2u(f16x2{static_cast<_Float16>(fmaf(v[2 * i], sc, -static_cast<float>(hp[0]))),
-                         static_cast<_Float16>(fmaf(v[2 * i + 1], sc, -static_cast<float>(hp[1])))});
-    }
-    hi = make_uint4(h[0], h[1], h[2], h[3]);
-    lo = make_uint4(l[0], l[1], l[2], l[3]);
-}
-
-// an infinite value has no lo part
-__device__ __forceinline__ uint32_t finite_lo(uint32_t h, uint32_t l) {
-    l = (h & 0x7fffu) == 0x7c00u ? l & 0xffff0000u : l;
-    return (h & 0x7fff0000u) == 0x7c000000u ? l & 0x0000ffffu : l;
-}
-__device__ __forceinline__ void drop_inf(const uint4 &h, uint4 &l) {
-    l = make_uint4(finite_lo(h.x, l.x), finite_lo(h.y, l.y), finite_lo(h.z, l.z), finite_lo(h.w, l.w));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4 mfma16(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, const f32x4 &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, make_uint2(a0, a1)),
+                                                     __builtin_bit_cast(s16x4, make_uint2(b0, b1)), c, 0, 0, 0);
 }
 
 template <int T, int MODE, int NT, int TT>
@@ -395,17 +348,14 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
         rp[t] = (t < OT ? a.w0 : a.w1) + row * a.rb;
     }
     f32x4 acc[TT][NT];
-    float limit[TT];  // 2^(15 - s) of the lane's token in each tile (0: no value yet)
 #pragma unroll
-    for (int i = 0; i < TT; ++i) {
-        limit[i] = 0.0f;
+    for (int i = 0; i < TT; ++i)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
 
     // x of a token tile's unit: read along the tokens' rows (32 lanes of a token, two tokens a request),
-    // turned in the wave's own LDS (slot c of token t at c ^ t) into lane (token n, elements 8g .. 8g+7 of
-    // every block).  A wave's LDS accesses complete in order, so it needs no waits of its own.
+    // turned in the wave's own LDS (slot c of token t at c ^ t) into lane (token n, the lane group's slots).
+    // A wave's LDS accesses complete in order, so it needs no waits of its own.
     f32x4 *turn = part + wave * (16 * 8 * kUnit);
     const int lt = lane >> 5, lc = lane & 31;
     auto load_x = [&](f32x4 (&x)[2 * kUnit], int i, int u) {
@@ -420,7 +370,7 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
         for (int p = 0; p < 2 * kUnit; ++p) turn[(2 * p + lt) * 32 + (lc ^ (2 * p + lt))] = x[p];
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int e = 0; e < 2 * kUnit; ++e) r[e] = turn[n * 32 + ((8 * (e >> 1) + 2 * g + (e & 1)) ^ n)];
+        for (int e = 0; e < 2 * kUnit; ++e) r[e] = turn[n * 32 + (Unit<T>::x_slot(e, g) ^ n)];
         __builtin_amdgcn_wave_barrier();
     };
     Unit<T> raw[NT];
@@ -432,10 +382,19 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
         load_x(ahead, 0, u);
     }
     for (; u < nunit; u += kDWaves) {  // uniform
-        uint4 B[NT][kUnit], B2[NT][Q6 ? kUnit : 1];
-        float dw[NT][kUnit];
+        u32x4 B[NT][kUnit];
+        float dw[NT][Unit<T>::kScales];
+        float dmax = 0.0f;
 #pragma unroll
-        for (int t = 0; t < NT; ++t) raw[t].operands(g, B[t], B2[t], dw[t]);
+        for (int t = 0; t < NT; ++t) {
+            raw[t].operands(g, B[t], dw[t]);
+            // (the packed values, not the floats they were made from, stay live)
+#pragma unroll
+            for (int j = 0; j < kUnit; ++j) asm("" : "+v"(B[t][j]));
+#pragma unroll
+            for (int j = 0; j < Unit<T>::kScales; j += 2) dmax = max3_abs(dw[t][j], dw[t][j + 1], dmax);
+        }
+        const bool winf = !(dmax <= 3.4e38f);  // (a scale that is NaN makes NaN either way)
         const int next = u + kDWaves;
         auto tile = [&](int i) {
             f32x4 x[2 * kUnit];
@@ -458,71 +417,56 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
             float am = 0.0f;
 #pragma unroll
             for (int e = 0; e < 2 * kUnit; ++e) am = max3_abs(x[e][2], x[e][3], max3_abs(x[e][0], x[e][1], am));
-            am = max_over_groups(am);
-            const bool inf = !(am <= 3.4e38f);
-            if (__any(am > limit[i])) {  // uniform, rare: new scales, the sums so far brought to them
-                asm volatile("");
-                float f = 1.0f;
-                if (am > limit[i]) {
-                    if (inf) {
-                        if (limit[i] == 0.0f) limit[i] = 32768.0f;
-                    } else {
-                        int ex;
-                        (void)frexpf(am, &ex);
-                        const float was = limit[i];
-                        limit[i] = ldexpf(1.0f, 15 - min(13 - ex, 120));
-                        if (was > 0.0f) f = was / limit[i];
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float fr = __shfl(f, 4 * g + r, 64);
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) acc[i][t][r] *= fr;
-                }
-            }
-            // 2^s: the exponents of limit and 2^s add up to 15 (no value yet: some finite number, against zeros)
-            const float sc = __builtin_bit_cast(float, (269u << 23) - __builtin_bit_cast(uint32_t, limit[i]));
-            auto blocks = [&](auto with_inf) {
-                [[maybe_unused]] f32x4 D6[NT];
+            if (__any(out_of_range(am) || winf)) {  // uniform, rare: as f32 values
 #pragma unroll
                 for (int j = 0; j < kUnit; ++j) {
-                    uint4 hi, lo;
-                    split8(x[2 * j], x[2 * j + 1], sc, hi, lo);
-                    uint4 hi2 = hi;  // against B2, which may be 0 where the weight is not: no infinite values
-                    if constexpr (decltype(with_inf)::value) {
-                        drop_inf(hi, lo);
-                        drop_inf(hi, hi2);
+                    if (!Q6 && kUnit * u + j >= nblk) break;  // uniform (its weights are not the row's)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        u32x4 b = B[t][j];
+                        asm volatile("" : "+v"(b));  // (the f32 values are not kept from tile to tile)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            acc[i][t] = mfma_f32(x[2 * j + (e >> 2)][e & 3],
+                                                 mul_rn(dw[t][Q6 ? 2 * j + (e >> 2) : j], bf16_at(b, e)), acc[i][t]);
                     }
-                    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (Q6) {  // d is the unit's: its blocks add up first
+                }
+                return;
+            }
+            const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) D6[t] = mfma_h(hi, B[t][j], j ? D6[t] : zero);
+            for (int j = 0; j < kUnit; ++j) {
+                u32x4 hi, mid, lo;
+                split3(x[2 * j], x[2 * j + 1], hi, mid, lo);
+                if constexpr (Q6) {
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) D6[t] = mfma_h(hi2, B2[t][j], D6[t]);
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) D6[t] = mfma_h(lo, B[t][j], D6[t]);
-                    } else {
+                    for (int s = 0; s < 2; ++s) {
                         f32x4 D[NT];
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) D[t] = mfma_h(hi, B[t][j], zero);
+                        for (int t = 0; t < NT; ++t) D[t] = mfma16(lo[2 * s], lo[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], zero);
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) D[t] = mfma_h(lo, B[t][j], D[t]);
+                        for (int t = 0; t < NT; ++t) D[t] = mfma16(mid[2 * s], mid[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], D[t]);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) D[t] = mfma16(hi[2 * s], hi[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], D[t]);
 #pragma unroll
                         for (int t = 0; t < NT; ++t)
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][j], D[t][r], acc[i][t][r]);
+                            for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][2 * j + s], D[t][r], acc[i][t][r]);
                     }
-                }
-                if constexpr (Q6) {
+                } else {
+                    f32x4 D[NT];
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) D[t] = mfma(lo, B[t][j], zero);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) D[t] = mfma(mid, B[t][j], D[t]);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) D[t] = mfma(hi, B[t][j], D[t]);
 #pragma unroll
                     for (int t = 0; t < NT; ++t)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][0], D6[t][r], acc[i][t][r]);
+                        for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][j], D[t][r], acc[i][t][r]);
                 }
-            };
-            if (__any(inf)) blocks(std::true_type{});  // uniform
-            else blocks(std::false_type{});
+            }
 #pragma unroll
             for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(acc[i][t]));  // (not sunk below the next tile)
         };
@@ -533,16 +477,11 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
     }
     __syncthreads();  // (the sums below take the LDS of the tiles)
 
-    // each wave's sums at their true scale; lane (row, g) of D holds tokens 4g .. 4g+3
+    // lane (row, g) of D holds tokens 4g .. 4g+3
 #pragma unroll
-    for (int i = 0; i < TT; ++i) {
-        const float inv = limit[i] > 0.0f ? limit[i] * 0x1p-15f : 1.0f;
-        f32x4 iv;
+    for (int i = 0; i < TT; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) iv[r] = __shfl(inv, 4 * g + r, 64);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) part[((wave * NT + t) * TT + i) * 64 + lane] = acc[i][t] * iv;
-    }
+        for (int t = 0; t < NT; ++t) part[((wave * NT + t) * TT + i) * 64 + lane] = acc[i][t];
     __syncthreads();
     const int rows = min(16 * OT, a.n - row0), toks = min(16 * TT, a.m - t0);
     for (int e = tid; e < 16 * OT * 16 * TT; e += kDThreads) {
@@ -571,44 +510,21 @@ hipError_t launch_rows(const DenseArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// The tiles of a launch: NT row tiles (of a SwiGLU: NT / 2 outputs') by TT token tiles per workgroup, one
-// workgroup on a CU at a time.  Measured, a round of workgroups takes about 2 us plus, per unit of a wave,
-// 2.1 (1 x 1), 3.3 (2 x 1), 3.2 (1 x 2), 4.6 (2 x 2), 6.6 (2 x 3) and 8.8 us (2 x 4): larger tiles split x and read the
-// weights for more products, smaller ones fill the chip.  The cheapest total is taken (Q8_0 [896, 4864] at 384
-// tokens: 168 workgroups of 2 x 4 tiles 44 us, 224 of 2 x 3 32 us).
-struct RowsPlan {
-    int nt, tt;
-    float us;
-};
-RowsPlan rows_plan(int n, int k, int m, bool swiglu) {
-    static constexpr struct {
-        int nt, tt;
-        float unit;
-    } kinds[] = {{1, 1, 2.1f}, {2, 1, 3.3f}, {1, 2, 3.2f}, {2, 2, 4.6f}, {2, 3, 6.6f}, {2, 4, 8.8f}};
-    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    const float units = static_cast<float>((k / 32 + kUnit * kDWaves - 1) / (kUnit * kDWaves));
-    RowsPlan best{0, 0, 0.0f};
-    for (const auto &c : kinds) {
-        if (swiglu && c.nt == 1) continue;
-        const int rows = 16 * c.nt / (swiglu ? 2 : 1), toks = 16 * c.tt;
-        const int64_t wgs = static_cast<int64_t>((n + rows - 1) / rows) * ((m + toks - 1) / toks);
-        const float us = static_cast<float>((wgs + cus - 1) / cus) * (2.0f + units * c.unit);
-        if (!best.nt || us < best.us) best = RowsPlan{c.nt, c.tt, us};
-    }
-    return best;
-}
+int cu_count() { return device_info().cu_count > 0 ? device_info().cu_count : 256; }
 
 template <int T, int MODE>
 hipError_t by_shape(const DenseArgs &a, hipStream_t s) {
-    const RowsPlan p = rows_plan(a.n, a.k, a.m, MODE == kSwiGLU);
+    const plan::Rows p = plan::rows(T, a.n, a.k, a.m, MODE == kSwiGLU, cu_count());
     if constexpr (MODE != kSwiGLU) {
         if (p.nt == 1) return p.tt == 1 ? launch_rows<T, MODE, 1, 1>(a, s) : launch_rows<T, MODE, 1, 2>(a, s);
+    }
+    if constexpr (T != T_Q6_K) {
+        if (p.tt == 4) return launch_rows<T, MODE, 2, 4>(a, s);
     }
     switch (p.tt) {
         case 1: return launch_rows<T, MODE, 2, 1>(a, s);
         case 2: return launch_rows<T, MODE, 2, 2>(a, s);
-        case 3: return launch_rows<T, MODE, 2, 3>(a, s);
-        default: return launch_rows<T, MODE, 2, 4>(a, s);
+        default: return launch_rows<T, MODE, 2, 3>(a, s);
     }
 }
 
@@ -628,11 +544,11 @@ bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const f
     const auto al = [](const void *p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & (m - 1)) == 0; };
     if (type == T_Q4_K) return k % 256 == 0 && rb % 16 == 0 && al(w0, 16) && (!w1 || al(w1, 16)) && al(x, 16);
     if (type != T_Q4_0 && type != T_Q5_0 && type != T_Q8_0 && type != T_Q6_K) return false;
-    // the per-element decoder reads 16-bit fields: 2-byte aligned blocks
+    // blocks are read at their 2-byte alignment
     return k % 32 == 0 && rb % 2 == 0 && al(w0, 2) && (!w1 || al(w1, 2)) && al(x, 16);
 }
 
-float dense_us(int n, int k, int m, bool swiglu) { return rows_plan(n, k, m, swiglu).us; }
+float dense_us(int type, int n, int k, int m, bool swiglu) { return plan::rows(type, n, k, m, swiglu, cu_count()).us; }
 
 hipError_t dense_matmul(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const float *x, float *y, int n,
                         int k, int m, int mode, hipStream_t s, const RouteCombine *combine) {

@@ -93,8 +93,8 @@ hipError_t mfma_down_routed(int type, const uint8_t *wd, size_t expert_bytes, si
                             hipStream_t s);
 
 // m > 1 rows of f32 activations (qlin_dense.hip), for fewer than kF32GemmMinRows rows or the other
-// formats: Q4_K on the bf16 matrix cores with x as bf16 hi + lo (x to about 2^-17 of itself, products
-// exact, f32 accumulation), the other formats on the f32 matrix cores with the reference's f32 operands.
+// formats, on the bf16 matrix cores with exact products and f32 accumulation: Q4_K with x as bf16 hi + lo (x
+// to about 2^-17 of itself), the other formats with all of x in three bf16 parts.
 // Mode 0 stores y[r, o], 1 adds into it, 2 writes act[r, o] = silu(gate . x_r) * (up . x_r) with w1 the up
 // matrix.
 bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, int in_dim);
@@ -138,7 +138,7 @@ hipError_t quantize_q8_1(const float *x, uint8_t *xq, int in_dim, int m, bool ra
 // layout the entry points accept.  gemm_us, dense_us: the estimated microseconds of gemm_f32 and of
 // dense_matmul (all formats but Q4_K), from which the dispatch chooses.
 float gemm_us(int n, int k, int m, bool swiglu);
-float dense_us(int n, int k, int m, bool swiglu);
+float dense_us(int type, int n, int k, int m, bool swiglu);
 hipError_t gemm_f32(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, float *y, int n,
                     int k, int m, int mode, hipStream_t s);
 hipError_t gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, float *y, int n, int k, int m,

@@ -88,5 +88,47 @@ inline Stream stream(const StreamFmt &f, bool swiglu, int rows, int K, int E, in
     return p;
 }
 
+// Several rows of activations: the formats' order in the tables below (ggml types Q4_0, Q5_0, Q8_0, Q6_K).
+inline int rows_format(int type) { return type == 2 ? 0 : type == 6 ? 1 : type == 8 ? 2 : type == 14 ? 3 : -1; }
+inline int64_t tiles(int n, int bn, int m, int bm) {
+    return static_cast<int64_t>((n + bn - 1) / bn) * ((m + bm - 1) / bm);
+}
+
+// The row products of qlin_dense.hip (rows_kernel): nt row tiles (of a SwiGLU: nt / 2 outputs') by tt token tiles
+// of 16 per workgroup, one workgroup on a CU at a time, whose 8 waves take units of 128 values of K in turn.
+// us is `base` plus, per round of workgroups, round + unit x (units of a wave): least squares of the logarithm over
+// the tiles of 36 shapes of each format (n 512 .. 32768, k 512 .. 16384, m 2 .. 700), 9-10% off in the mean; the
+// kernel it picks is 0.2% slower in the mean than the fastest, 13% at most.  Larger tiles split x and read the
+// weights for more products, smaller ones fill the chip.  Q6_K has no 2 x 4 tiles (they spill: 8.0 us a unit, as
+// much per product as 2 x 3's 5.7).
+struct Rows {
+    int nt = 0, tt = 0;
+    float us = 0.0f;
+};
+inline Rows rows(int type, int n, int k, int m, bool swiglu, int cus) {
+    static constexpr int nt[6] = {1, 2, 1, 2, 2, 2}, tt[6] = {1, 1, 2, 2, 3, 4};
+    static constexpr struct {
+        float base, round[6], unit[6];
+    } costs[4] = {{0.75f, {0.95f, 1.55f, 1.4f, 2.4f, 3.1f, 3.3f}, {1.45f, 1.98f, 2.42f, 3.1f, 4.1f, 5.2f}},
+                  {0.8f, {0.9f, 1.6f, 1.55f, 2.3f, 2.9f, 3.6f}, {1.63f, 2.31f, 2.58f, 3.5f, 4.6f, 5.6f}},
+                  {1.7f, {0.9f, 1.1f, 1.15f, 1.85f, 2.2f, 2.85f}, {1.53f, 2.39f, 2.62f, 3.5f, 4.5f, 5.7f}},
+                  {1.45f, {0.95f, 1.15f, 1.25f, 1.4f, 2.45f, 0.0f}, {1.83f, 3.2f, 2.86f, 4.55f, 5.7f, 0.0f}}};
+    const int f = rows_format(type);
+    Rows best;
+    if (f < 0) return best;
+    const float units = static_cast<float>((k / 32 + 31) / 32);
+    for (int i = 0; i < (f == 3 ? 5 : 6); ++i) {
+        if (swiglu && nt[i] == 1) continue;
+        const int64_t wgs = tiles(n, 16 * nt[i] / (swiglu ? 2 : 1), m, 16 * tt[i]);
+        const float us = costs[f].base + static_cast<float>((wgs + cus - 1) / cus) * (costs[f].round[i] + units * costs[f].unit[i]);
+        if (!best.nt || us < best.us) {
+            best.nt = nt[i];
+            best.tt = tt[i];
+            best.us = us;
+        }
+    }
+    return best;
+}
+
 }  // namespace plan
 }  // namespace qlin

@@ -201,8 +201,8 @@ def test_gemv_several_rows(qtype, m):
     (Q6_K, 300, 512, 129)])
 def test_matmul_rows_f32_matrix_cores(qtype, out_dim, in_dim, m):
     """m > 1 rows (launch_quant_matmul, kernel.cu:1254-1279) on the matrix cores: below 64 rows, Q4_K on
-    the bf16 ones (x as bf16 hi + lo) and the other formats on the f32 ones; from 64 rows, Q4_K and Q6_K
-    on the prefill GEMM (fp16, x as scaled hi + lo).  Row tails (out_dim % 16, and of the GEMM's 256-row
+    the bf16 ones with x as bf16 hi + lo, from 64 rows on its prefill GEMM (fp16, x as scaled hi + lo); the
+    other formats here with x in three bf16 parts.  Row tails (out_dim % 16, and of the GEMM's 256-row
     tiles), fewer and more chunks than waves, a partial last chunk (K / 32 not a multiple of 8), token
     tails within and across 64-token tiles, and every format."""
     w, rb, vals = qgen.random_matrix(qtype, out_dim, in_dim, seed=out_dim + m + qtype)
@@ -237,8 +237,7 @@ def test_matmul_add_rows(qtype, m):
                                             (Q8_0, 96, 512, 3), (Q6_K, 2816, 2048, 16), (Q5_0, 100, 160, 4)])
 def test_swiglu_rows(qtype, ffn, hid, m):
     """act[r] = silu(Wg x[r]) * (Wu x[r]) for a batch: C5's shared experts ([2816, 2048] Q4_K gate/up,
-    16 tokens), a short batch, one row (the single-row kernel) and the other formats on the f32
-    matrix-core kernel."""
+    16 tokens), a short batch, one row (the single-row kernel) and the other formats."""
     wg, rb, _ = qgen.random_matrix(qtype, ffn, hid, seed=ffn + m)
     wu, _, _ = qgen.random_matrix(qtype, ffn, hid, seed=ffn + m + 1)
     x = qgen.random_x(m, hid, seed=m + 3)
@@ -547,8 +546,7 @@ BLOCK_ROWS = [  # (type, N, K, m): few rows and short K (a unit of blocks cut sh
 @pytest.mark.parametrize("mode", ["store", "add", "swiglu"])
 @pytest.mark.parametrize("qtype,N,K,m", BLOCK_ROWS)
 def test_rows_of_f32(qtype, N, K, m, mode):
-    """Several rows of f32 activations through the split-fp16 kernels (quant_matmul, its add form, the SwiGLU
-    rows): against the f64 oracle, each output within 2e-5 of its own sum |w||x| (the bound of the other
+    """Several rows of f32 activations (quant_matmul, its add form, the SwiGLU rows): against the f64 oracle, each output within 2e-5 of its own sum |w||x| (the bound of the other
     f32 paths) and normwise 1e-5."""
     w, rb, vals = qgen.random_matrix(qtype, N, K, seed=K + m)
     x = qgen.random_x(m, K, seed=N + m)
@@ -612,6 +610,64 @@ def test_rows_of_f32_token_scales(qtype, N, m):
         assert np.isnan(got[t][wk == 0]).all()
         assert (got[t][wk != 0] == np.sign(wk[wk != 0]) * x[t, k]).all()
     assert np.isnan(got[17]).all()
+
+
+def _zero_weight(qtype, w, rb, vals, rows, k):
+    """Sets element k (k % 32 < 16; Q6_K: 64 <= k < 80) of the rows to weight 0."""
+    b = w.reshape(-1, rb)
+    e = k % 32
+    if qtype == Q8_0:
+        b[rows, k // 32 * 34 + 2 + e] = 0
+    elif qtype == Q4_0:
+        i = k // 32 * 18 + 2 + e
+        b[rows, i] = (b[rows, i] & 0xf0) | 8
+    elif qtype == Q5_0:
+        i = k // 32 * 22
+        b[rows, i + 6 + e] &= 0xf0
+        b[rows, i + 2 + e // 8] |= 1 << e % 8
+    else:
+        b[rows, e] &= 0x0f
+        b[rows, 128 + e] = (b[rows, 128 + e] & 0xcf) | 0x20
+    vals[rows, k] = 0.0
+
+
+WIDE_ROWS = [(Q8_0, 300, 70), (Q6_K, 300, 40), (Q5_0, 300, 20), (Q4_0, 300, 9)]
+
+
+@pytest.mark.parametrize("qtype,N,m", WIDE_ROWS)
+def test_rows_of_f32_over_the_whole_range(qtype, N, m):
+    """Values up to the largest finite one and down to the smallest normal ones, in tokens of their own and
+    beside one another, with weight 0 under the largest in every second row: each output within the bound of
+    its own sum |w||x|, as f32 products give it (a scale shared by a token's values would overflow, or round
+    the small ones away).  An infinite value beside large finite ones: infinite with its weight's sign."""
+    K, k0 = 1024, 77
+    w, rb, vals = qgen.random_matrix(qtype, N, K, seed=295, scale=1e-5)
+    _zero_weight(qtype, w, rb, vals, np.arange(0, N, 2), k0)
+    rng = np.random.default_rng(296)
+    x = rng.standard_normal((m, K)).astype(np.float32)
+    x[0] *= np.float32(5e37)
+    x[1, k0] = np.finfo(np.float32).max
+    x[2] *= np.float32(1e-6)
+    x[2, k0] = 1e6
+    x[3] *= np.logspace(30, -30, K).astype(np.float32)
+    x[4] *= np.float32(1e-36)
+    x[5, :128] *= np.float32(1e37)
+    x[5, 128:] *= np.float32(1e-36)
+    x[5, 512:640] = 0.0
+    x[6] *= np.float32(1e30)
+    x[6, k0] = -np.inf
+    banner(f"rows whole range type={qtype} N={N} m={m}")
+    yd = empty_f32(m, N)
+    qlin.quant_matmul(qtype, dev(w), rb, dev(x), yd, N, K, m)
+    got = host(yd)
+    fine = np.r_[0:6, 7:m]
+    ref = orc.matmul_f64(qtype, w, rb, x[fine], N, K)
+    scale = np.abs(x[fine].astype(np.float64)) @ np.abs(vals.astype(np.float64)).T
+    err = np.abs(got[fine] - ref) / scale
+    assert np.isfinite(got[fine]).all() and err.max() <= COND, (err.max(axis=1), np.isfinite(got[fine]).all(axis=1))
+    w0 = vals[:, k0].astype(np.float64)
+    assert np.isnan(got[6][w0 == 0]).all()
+    assert (got[6][w0 != 0] == -np.sign(w0[w0 != 0]) * np.inf).all()
 
 
 @pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 14400, 1088, 257), (Q5_0, 14400, 1024, 130), (Q4_0, 70, 96, 5),
