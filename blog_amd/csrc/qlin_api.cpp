@@ -313,7 +313,7 @@ int qlin_launch_quant_swiglu_rows(int type, const uint8_t *wg, const uint8_t *wu
     if (!work) return QLIN_OK;
     if (m > 1 && g_rb == u_rb && (type == QLIN_TYPE_Q4_0 || type == QLIN_TYPE_Q5_0 || type == QLIN_TYPE_Q8_0) &&
         (!qlin::dense_ok(type, wg, wu, g_rb, x, in_dim) ||
-         qlin::gemm_us(ffn_dim, in_dim, m, true) < qlin::dense_us(type, ffn_dim, in_dim, m, true)))
+         qlin::gemm_us(type, false, ffn_dim, in_dim, m, true) < qlin::dense_us(type, ffn_dim, in_dim, m, true)))
         return launched(qlin::gemm_f32(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));
     if (m > 1 && g_rb == u_rb && qlin::dense_ok(type, wg, wu, g_rb, x, in_dim))
         return launched(qlin::dense_matmul(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));

@@ -5,35 +5,37 @@
 //   y[r, o]  =     sum over 32-blocks of the Q8_1 block dots      (kernel.cu:2305-2402, quant_matmul_q8_1)
 //   act[r, o] = g / (1 + expf(-g)) * u, g, u the rows of two matrices (SharedExperts.cpp:34-40)
 //
-// Operands (v_mfma_f32_16x16x32_f16: products exact, f32 accumulation).
-//   A (activations): a token's values times a power of two 2^s, split into hi = fp16(x 2^s) and
-//     lo = fp16(x 2^s - hi), which together hold x 2^s to 2^-22 of its value down to 2^-16 of the
-//     token's largest; two MFMAs into one accumulator.  s comes from the token's largest magnitude so
-//     far (in [2^12, 2^13) after scaling), and only a value 4 times that or more changes it: then that
-//     token's sums are rescaled, exactly, before the step that brought it.  The result takes 2^-s at the
-//     end.  A Q8_1 activation is the value d8 q, its fp16 pair formed the same way (128 d8 bounds it).
-//   B (weights): q less its offset, an integer exact in fp16; the block's d by one fma per output.
+// Operands, A the activations and B the weights, all products exact, f32 accumulation.
+//   f32 activations: v_mfma_f32_16x16x32_bf16, x in its three bf16 parts (qlin_bf16x3.hpp), the weights as
+//     integers; the block's d by one fma per output.  A workgroup that meets a value that does not fit the
+//     parts computes its tile again at the end, as f32 values on v_mfma_f32_16x16x4_f32.
+//   Q8_1 activations: v_mfma_f32_16x16x32_f16 on integers on both sides, so a block's dot is exact; its
+//     scales d8 and d by a product and an fma per output.
 //
 // Tiling.  A workgroup of 8 waves computes BM tokens x BN weight rows in steps of 64 values of K.  Both
-// operands of a step are staged in LDS once per workgroup -- each weight decoded once for all BM
-// tokens, each activation split once for all BN rows -- in the MFMA lane layout, two buffers.  The
-// waves form a WM x WN grid, each MT x NT tiles of 16 x 16.  Between two barriers waves 0-3 (one per
-// SIMD) multiply step k and then stage their share of step k + 1, while waves 4-7 stage theirs of
-// step k + 1 and then multiply step k, so that one half's matrix instructions run beside the other's
-// vector ones.  Global loads are one step ahead (activations, from L2) and two (weights).
+// operands of a step are staged in LDS once per workgroup, in the MFMA lane layout, two buffers: each weight
+// decoded once for all BM tokens; f32 activations as they are (three parts would not fit beside the weights),
+// split by the WN waves that read them.  The waves form a WM x WN grid, each MT x NT tiles of 16 x 16.  Between
+// two barriers waves 0-3 (one per SIMD) multiply step k and then stage their share of step k + 1, while waves
+// 4-7 stage theirs of step k + 1 and then multiply step k, so that one half's matrix instructions run beside the
+// other's vector ones.  Global loads are one step ahead (activations, from L2) and two (weights).
 //
 // Slots of the LDS planes are permuted within a row group by an XOR with the k-group (A) or the chunk
 // (B), so that the staging writes and the fragment reads both spread over the banks.
 //
-// Measured (f32 activations): Q8_0 [14336, 4096] at 512 tokens 1738 -> 177 us (340 TFLOP/s) and Q4_0
-// [18944, 3584] at 203 tokens 618 -> 133 us against the f32 matrix cores with the weights decoded per 16
-// tokens; Q8_1 activations, Q8_0 [14336, 4096] at 512 tokens 315 -> 165 us against the 64-token tiles
-// that scale every block's products twice.  Matrix cores, vector ALU and LDS are each busy 35-45% of
-// the time: what bounds it is the step's chain (barrier, fragment reads, products, staging writes).
+// Measured (f32 activations): Q8_0 [14336, 4096] at 512 tokens 1746 -> 181 us and Q4_0 [18944, 3584] at 203 tokens
+// 618 -> 149 us against the f32 matrix cores with the weights decoded per 16 tokens (an fp16 pair of x under a
+// scale per token: 155 and 132 us, but not exact); Q8_1 activations, Q8_0 [14336, 4096] at 512 tokens 303 -> 121 us
+// against the 64-token tiles (155 with d8 q as an fp16 pair).  What bounds it: the step's chain (barrier, reads,
+// splits, products, staging writes); per step and SIMD the large tiles' vector instructions take about 3400
+// cycles, the matrix ones 3100, of 6500.
 //
 // Blocks and rows are only 2-byte aligned in general; weights are read as wide loads at that alignment.
+#include "qlin_bf16x3.hpp"
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
+#include "qlin_mfma.hpp"
+#include "qlin_plan.hpp"
 #include "qlin_values8.hpp"
 
 #include <type_traits>
@@ -43,28 +45,28 @@ namespace {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 enum : int { kStore = 0, kAdd = 1, kSwiGLU = 2 };
 
-constexpr int kWaves = 8, kThreads = kWaves * 64, kStep = 64;
+constexpr int kWaves = 8, kThreads = kWaves * 64;
 
-template <int MT_, int NT_, int WM_, int WN_>
+template <int MT_, int NT_, int WM_, int WN_, int HT_>
 struct Geo {
+    static constexpr int HT = HT_;  // tiles multiplied before the ones before them are scaled
     static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = WN_;
     static constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN;
     static constexpr int waves = MT * NT > 8 ? 2 : 4;  // per SIMD: two workgroups on a CU where LDS has room for them
     static_assert(WM * WN == kWaves, "8 waves");
 };
 
-// LDS, in uint4: two step buffers (hi and lo planes, weights, block scales, rescale factors), then the
-// tokens' final scales and the steps that rescale.
-template <class G>
+// LDS, in uint4: two step buffers (activations: f32 values 0..3 and 4..7 of a lane's 8, or fp16 and the
+// blocks' scales; weights; their block scales), then a flag.
+template <class G, bool Q81>
 struct Lds {
     static constexpr int a = G::BM / 16 * 2 * 64, b = G::BN / 16 * 2 * 64;
-    static constexpr int hi = 0, lo = a, w = 2 * a, dw = w + b, fac = dw + 2 * G::BN / 4;
-    static constexpr int buf = fac + G::BM / 4;
-    static constexpr int inv = 2 * buf, flag = inv + G::BM / 4, total = flag + 1;
+    static constexpr int x0 = 0, x1 = a, w = Q81 ? a : 2 * a, dw = w + b, dx = dw + 2 * G::BN / 4;
+    static constexpr int buf = dx + (Q81 ? 2 * G::BM / 4 : 0);
+    static constexpr int flag = 2 * buf, total = flag + 1;
     static constexpr size_t bytes = total * sizeof(uint4);
     static_assert(bytes <= 160 * 1024, "fits the CU's LDS");
 };
@@ -77,7 +79,7 @@ struct GemmArgs {
     int n, m, k;
 };
 
-__device__ __forceinline__ f32x4 mfma(const uint4 &a, const uint4 &b, const f32x4 &c) {
+__device__ __forceinline__ f32x4 mfma_h(const u32x4 &a, const u32x4 &b, const f32x4 &c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 __device__ __forceinline__ uint32_t h2u(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
@@ -89,6 +91,13 @@ __device__ __forceinline__ f16x2 splat(float v) {
 // bytes (b0, 0x64, b1, 0x64) or (b2, .., b3, ..) of v: the fp16 pair 1024 + byte
 __device__ __forceinline__ f16x2 bytes_lo(uint32_t v) { return u2h(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)); }
 __device__ __forceinline__ f16x2 bytes_hi(uint32_t v) { return u2h(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)); }
+// fp16 integers of 8 bytes less off - 1024
+__device__ __forceinline__ u32x4 minus8(uint32_t a, uint32_t b, f16x2 off) {
+    return u32x4{h2u(bytes_lo(a) + off), h2u(bytes_hi(a) + off), h2u(bytes_lo(b) + off), h2u(bytes_hi(b) + off)};
+}
+__device__ __forceinline__ u32x4 f16_of_i8(uint32_t a, uint32_t b) {
+    return minus8(a ^ 0x80808080u, b ^ 0x80808080u, splat(-1152.0f));
+}
 
 // Consumes a row of sums: pure arithmetic is otherwise sunk below the next products, whose results then
 // all stay live.
@@ -96,75 +105,6 @@ template <int NT>
 __device__ __forceinline__ void pin(f32x4 (&v)[NT]) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(v[t]));
-}
-
-// ---- activations ---------------------------------------------------------------------------------
-
-// hi and lo parts of 8 values times sc (a power of two), or of 8 fp16 integers times sc: two
-// mixed-precision fmas a value
-template <class V>
-__device__ __forceinline__ void split8(const V (&v)[8], float sc, uint4 &hi, uint4 &lo) {
-    uint32_t h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float a = static_cast<float>(v[2 * i]), b = static_cast<float>(v[2 * i + 1]);
-        h[i] = h2u(f16x2{static_cast<_Float16>(fmaf(a, sc, 0.0f)), static_cast<_Float16>(fmaf(b, sc, 0.0f))});
-        asm("" : "+v"(h[i]));  // one packed value (its halves would otherwise be formed twice)
-        const f16x2 hp = u2h(h[i]);
-        l[i] = h2u(f16x2{static_cast<_Float16>(fmaf(a, sc, -static_cast<float>(hp[0]))),
-                         static_cast<_Float16>(fmaf(b, sc, -static_cast<float>(hp[1])))});
-    }
-    hi = make_uint4(h[0], h[1], h[2], h[3]);
-    lo = make_uint4(l[0], l[1], l[2], l[3]);
-}
-
-// an infinite value has no lo part
-__device__ __forceinline__ uint32_t finite_lo(uint32_t h, uint32_t l) {
-    l = (h & 0x7fffu) == 0x7c00u ? l & 0xffff0000u : l;
-    return (h & 0x7fff0000u) == 0x7c000000u ? l & 0x0000ffffu : l;
-}
-__device__ __forceinline__ void drop_inf(const uint4 &h, uint4 &l) {
-    l = make_uint4(finite_lo(h.x, l.x), finite_lo(h.y, l.y), finite_lo(h.z, l.z), finite_lo(h.w, l.w));
-}
-
-// the largest of v over 8 lanes in a row (v >= 0, whose bits order as it does)
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_bits(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float max_of_8(float v) {
-    uint32_t b = __builtin_bit_cast(uint32_t, v);
-    b = max(b, dpp_bits<0xb1>(b));
-    b = max(b, dpp_bits<0x4e>(b));
-    b = max(b, dpp_bits<0x141>(b));
-    return __builtin_bit_cast(float, b);
-}
-// A token's scale 2^s, held as the magnitude 2^(15 - s) from which it has to change (0: no value yet).
-struct Scale {
-    float limit = 0.0f;
-    // 2^s: the exponents of limit and 2^s add up to 15 (for no value yet some finite number, against zeros)
-    __device__ __forceinline__ float sc() const {
-        return __builtin_bit_cast(float, (269u << 23) - __builtin_bit_cast(uint32_t, limit));
-    }
-    // the factor by which the token's sums so far change for a step whose largest magnitude is am
-    __device__ __forceinline__ float step(float am) {
-        if (!(am > limit)) return 1.0f;
-        if (!(am <= 3.4e38f)) {  // not finite: the result will not be either
-            if (limit == 0.0f) limit = 32768.0f;
-            return 1.0f;
-        }
-        int ex;
-        (void)frexpf(am, &ex);
-        const float was = limit;
-        limit = ldexpf(1.0f, 15 - min(13 - ex, 120));
-        return was > 0.0f ? was / limit : 1.0f;
-    }
-};
-// max(|a|, |b|, c) in one instruction
-__device__ __forceinline__ float max3_abs(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
 }
 
 // ---- weights -------------------------------------------------------------------------------------
@@ -201,20 +141,16 @@ template <> struct WRaw<T_Q4_0> {
     }
 };
 
-// fp16 integers of 8 bytes less off
-__device__ __forceinline__ uint4 minus8(uint32_t a, uint32_t b, f16x2 off) {
-    return make_uint4(h2u(bytes_lo(a) + off), h2u(bytes_hi(a) + off), h2u(bytes_lo(b) + off), h2u(bytes_hi(b) + off));
-}
-// bits 0..3 of b to bit 4 of bytes 0..3
-__device__ __forceinline__ uint32_t bit4_of_bytes(uint32_t b) { return (__umul24(b & 0xfu, 0x204081u) & 0x01010101u) << 4; }
-
-// Elements 8g .. 8g+7 of the block for g = 0..3 through put(g, values).
-template <int FMT, class Put>
+// Elements 8g .. 8g+7 of the block for g = 0..3 through put(g, values): fp16 beside Q8_1 activations, else bf16.
+template <int FMT, bool F16, class Put>
 __device__ __forceinline__ void decode(const WRaw<FMT> &r, Put put) {
     if constexpr (FMT == T_Q8_0) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-            put(g, minus8(r.q[g >> 1][2 * (g & 1)] ^ 0x80808080u, r.q[g >> 1][2 * (g & 1) + 1] ^ 0x80808080u, splat(-1152.0f)));
+        for (int g = 0; g < 4; ++g) {
+            const uint32_t a = r.q[g >> 1][2 * (g & 1)], b = r.q[g >> 1][2 * (g & 1) + 1];
+            put(g, F16 ? f16_of_i8(a, b) : bf16_of_i8(a, b));
+            if constexpr (!F16) __builtin_amdgcn_sched_barrier(0);  // (8 floats live at a time)
+        }
     } else {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {  // low nibbles: elements 0..15, high: 16..31
@@ -224,14 +160,16 @@ __device__ __forceinline__ void decode(const WRaw<FMT> &r, Put put) {
                 a |= bit4_of_bytes(r.qh >> (8 * g));
                 b |= bit4_of_bytes(r.qh >> (8 * g + 4));
             }
-            put(g, minus8(a, b, splat(FMT == T_Q5_0 ? -1040.0f : -1032.0f)));
+            constexpr float off = FMT == T_Q5_0 ? 16.0f : 8.0f;
+            put(g, F16 ? minus8(a, b, splat(-1024.0f - off)) : bf16_of_u8(a, b, off));
+            if constexpr (!F16) __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
 
 template <int FMT, bool Q81, int MODE, class G>
 __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs a) {
-    using L = Lds<G>;
+    using L = Lds<G, Q81>;
     constexpr int MT = G::MT, NT = G::NT, BM = G::BM, BN = G::BN;
     constexpr int kOut = MODE == kSwiGLU ? BN / 2 : BN;  // output columns per workgroup
     static_assert(MODE != kSwiGLU || NT % 2 == 0, "gate and up tiles in pairs");
@@ -245,7 +183,7 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
     const int nblk = a.k / 32, nstep = (nblk + 1) / 2;
     const bool odd = nblk & 1;  // uniform: the last step has one block
 
-    auto fbuf = [&](int at) { return reinterpret_cast<float *>(lds + at); };
+    int *const again = reinterpret_cast<int *>(lds + L::flag);  // some value does not fit the parts
 
     // ---- staging: activations.  Lane q of a token's 8 takes values 8q .. 8q+7 of the step.
     constexpr int XP = (BM * 8 + kThreads - 1) / kThreads;  // tokens per thread
@@ -253,10 +191,9 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
     constexpr int XB = Q81 ? 36 : 128;  // bytes of a block
     const int xq8 = tid & 7, xchunk = xq8 >> 2, xg = xq8 & 3;
     const bool xlive = XAll || tid < BM * 8;
-    using XVec = std::conditional_t<Q81, uint2, float4>;
+    using XVec = std::conditional_t<Q81, uint2, f32x4>;
     XVec xv[XP][Q81 ? 1 : 2];
     uint32_t xds[Q81 ? XP : 1];  // a Q8_1 block's d and s
-    Scale xs[XP];
     const uint8_t *xrow[XP];
 #pragma unroll
     for (int p = 0; p < XP; ++p) {
@@ -282,48 +219,25 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
     };
     auto stage_x = [&](int step, uint4 *buf) {
         if (!xlive) return;
+        const bool none = odd && step == nstep - 1 && xchunk;  // the missing last block: zeros
 #pragma unroll
         for (int p = 0; p < XP; ++p) {
             const int tok = p * (kThreads / 8) + (tid >> 3);
             const int at = ((tok >> 4) * 2 + xchunk) * 64 + xg * 16 + ((tok & 15) ^ (2 * xq8));
-            if (odd && step == nstep - 1) {  // uniform
-                asm volatile("");  // (a branch, not selects in every step)
-                if (!xchunk) {
-                } else if constexpr (Q81) {
-                    xds[p] = 0u;
-                } else {
-                    xv[p][0] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    xv[p][1] = xv[p][0];
+            if constexpr (Q81) {
+                buf[L::x0 + at] = __builtin_bit_cast(uint4, f16_of_i8(xv[p][0].x, xv[p][0].y));
+                if (xg == 0)
+                    reinterpret_cast<float *>(buf + L::dx)[xchunk * BM + tok] = none ? 0.0f : f16_bits_to_f32(xds[p] & 0xffffu);
+            } else {
+                if (odd && step == nstep - 1) {  // uniform
+                    asm volatile("");            // (a branch, not selects in every step)
+                    if (none) xv[p][0] = xv[p][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 }
-            }
-            uint4 hi, lo;
-            float am;
-            if constexpr (Q81) {
-                am = fabsf(f16_bits_to_f32(xds[p] & 0xffffu)) * 128.0f;
-            } else {
-                const float4 u = xv[p][0], v = xv[p][1];
-                am = max3_abs(v.z, v.w, max3_abs(v.x, v.y, max3_abs(u.z, u.w, max3_abs(u.x, u.y, 0.0f))));
-            }
-            am = max_of_8(am);
-            const float f = xs[p].step(am);
-            const float sc = xs[p].sc();
-            if constexpr (Q81) {
-                const uint32_t q[2] = {xv[p][0].x ^ 0x80808080u, xv[p][0].y ^ 0x80808080u};
-                const f16x2 off = splat(-1152.0f);
-                const f16x2 e[4] = {bytes_lo(q[0]) + off, bytes_hi(q[0]) + off, bytes_lo(q[1]) + off, bytes_hi(q[1]) + off};
-                const _Float16 v[8] = {e[0][0], e[0][1], e[1][0], e[1][1], e[2][0], e[2][1], e[3][0], e[3][1]};
-                split8(v, f16_bits_to_f32(xds[p] & 0xffffu) * sc, hi, lo);
-            } else {
-                const float4 u = xv[p][0], v = xv[p][1];
-                const float fv[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-                split8(fv, sc, hi, lo);
-            }
-            if (!(am <= 3.4e38f)) drop_inf(hi, lo);
-            buf[L::hi + at] = hi;
-            buf[L::lo + at] = lo;
-            if (xq8 == 0) {
-                reinterpret_cast<float *>(buf + L::fac)[tok] = f;
-                if (f != 1.0f) reinterpret_cast<int *>(lds + L::flag)[step & 1] = step;
+                const f32x4 u = xv[p][0], v = xv[p][1];
+                const float am = max3_abs(v[2], v[3], max3_abs(v[0], v[1], max3_abs(u[2], u[3], max3_abs(u[0], u[1], 0.0f))));
+                if (out_of_range(am)) *again = 1;
+                buf[L::x0 + at] = __builtin_bit_cast(uint4, u);
+                buf[L::x1 + at] = __builtin_bit_cast(uint4, v);
             }
         }
     };
@@ -355,21 +269,24 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
 #pragma unroll
         for (int p = 0; p < WP; ++p) w[p].load(wrow[p] + off);
     };
-    auto stage_w = [&](const WRaw<FMT> (&w)[WP], uint4 *buf) {
+    auto stage_w = [&](const WRaw<FMT> (&w)[WP], int step, uint4 *buf) {
         if (!wlive) return;
 #pragma unroll
         for (int p = 0; p < WP; ++p) {
             const int r = p * (kThreads / 2) + (tid >> 1);
             const int at = ((r >> 4) * 2 + whalf) * 64 + ((r & 15) ^ (8 * whalf));
-            decode<FMT>(w[p], [&](int gg, const uint4 &v) { buf[L::w + at + 16 * gg] = v; });
-            reinterpret_cast<float *>(buf + L::dw)[whalf * BN + r] = f16_bits_to_f32(w[p].d);
+            decode<FMT, Q81>(w[p], [&](int gg, const u32x4 &v) { buf[L::w + at + 16 * gg] = __builtin_bit_cast(uint4, v); });
+            // (the missing last block: 0, as its activations)
+            reinterpret_cast<float *>(buf + L::dw)[whalf * BN + r] =
+                odd && step == nstep - 1 && whalf ? 0.0f : f16_bits_to_f32(w[p].d);
+            if (!Q81 && (w[p].d & 0x7c00u) == 0x7c00u) *again = 1;
         }
     };
     // The next steps' loads go out behind a step's staging.  Past the last step it stages the last blocks
     // again, into a buffer that is not read any more.
     auto stage = [&](WRaw<FMT> (&w)[WP], int step) {
         uint4 *buf = lds + (step & 1) * L::buf;
-        stage_w(w, buf);
+        stage_w(w, step, buf);
         load_w(w, step + 2);
         stage_x(step, buf);
         load_x(step + 1);
@@ -381,73 +298,109 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // One row of tiles at a time; the fragments of two rows on are read, and the row before's products
-    // scaled, next to its MFMAs.
+    // A row of HT tiles (of one chunk) at a time: the operands of the next one are read or split, and the row
+    // before's products scaled, next to its MFMAs.
+    constexpr int HT = G::HT, H = NT / HT;
+    static_assert(NT % HT == 0, "whole groups of tiles");
+    struct Raw {  // a lane's values of a tile row, and its Q8_1 tokens' scales
+        u32x4 v[Q81 ? 1 : 2];
+        f32x4 dx;
+    };
+    struct Operands {
+        u32x4 part[Q81 ? 1 : 3];  // smallest first
+        f32x4 dx;
+    };
+    auto load_raw = [&](const uint4 *buf, int c, int i) {
+        const int at = ((wm * MT + i) * 2 + c) * 64 + g * 16 + (n ^ (8 * c + 2 * g));
+        Raw r{};
+        r.v[0] = __builtin_bit_cast(u32x4, buf[L::x0 + at]);
+        if constexpr (Q81)
+            r.dx = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(buf + L::dx) + c * BM + (wm * MT + i) * 16 + 4 * g);
+        else
+            r.v[1] = __builtin_bit_cast(u32x4, buf[L::x1 + at]);
+        return r;
+    };
+    auto operands = [&](const Raw &r) {
+        Operands o;
+        if constexpr (Q81) {
+            o.part[0] = r.v[0];
+            o.dx = r.dx;
+        } else {
+            split3(__builtin_bit_cast(f32x4, r.v[0]), __builtin_bit_cast(f32x4, r.v[1]), o.part[2], o.part[1], o.part[0]);
+        }
+        return o;
+    };
+    struct Cols {
+        u32x4 b[HT];
+        float dw[HT];
+    };
+    auto load_cols = [&](const uint4 *buf, int c, int h) {
+        Cols v;
+#pragma unroll
+        for (int t = 0; t < HT; ++t) {
+            const int tile = wn * NT + h * HT + t;
+            v.b[t] = __builtin_bit_cast(u32x4, buf[L::w + (tile * 2 + c) * 64 + g * 16 + (n ^ (8 * c))]);
+            v.dw[t] = reinterpret_cast<const float *>(buf + L::dw)[c * BN + tile * 16 + n];
+        }
+        return v;
+    };
     auto multiply = [&](int step) {
         const uint4 *buf = lds + (step & 1) * L::buf;
-        const int flag = reinterpret_cast<const int *>(lds + L::flag)[step & 1];
-        struct Row {
-            uint4 h, l;
-        };
-        auto load_row = [&](int c, int i) {
-            const int at = ((wm * MT + i) * 2 + c) * 64 + g * 16 + (n ^ (8 * c + 2 * g));
-            return Row{buf[L::hi + at], buf[L::lo + at]};
-        };
-        struct Cols {
-            uint4 b[NT];
-            float dw[NT];
-        };
-        auto load_cols = [&](int c) {
-            Cols v;
+        constexpr int N = 2 * H * MT;  // rows: row v is tile row v % MT of column group v / MT % H of chunk v / MT / H
+        Raw raw[MT];
+        Operands x[MT];
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                v.b[t] = buf[L::w + ((wn * NT + t) * 2 + c) * 64 + g * 16 + (n ^ (8 * c))];
-                v.dw[t] = reinterpret_cast<const float *>(buf + L::dw)[c * BN + (wn * NT + t) * 16 + n];
+        for (int i = 0; i < MT; ++i) raw[i] = load_raw(buf, 0, i);
+        Cols col = load_cols(buf, 0, 0), next = col;
+        x[0] = operands(raw[0]);
+        f32x4 d[2][HT], dxp = {};
+        float dwp[HT] = {};  // the scales of the row before
+        auto scale = [&](int v) {
+            const int i = v % MT, h = v / MT % H;
+            f32x4 s[HT];
+#pragma unroll
+            for (int t = 0; t < HT; ++t) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float p = Q81 ? d[v & 1][t][r] * dxp[r] : d[v & 1][t][r];
+                    s[t][r] = fmaf(dwp[t], p, acc[i][h * HT + t][r]);
+                }
             }
-            return v;
-        };
-        Cols col = load_cols(0), col1;
-        Row row[3] = {load_row(0, 0), load_row(MT > 1 ? 0 : 1, MT > 1 ? 1 : 0), Row{}};
-        if (__builtin_amdgcn_readfirstlane(flag) == step) {  // uniform
+            pin(s);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                const f32x4 f = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(buf + L::fac) +
-                                                                 (wm * MT + i) * 16 + 4 * g);
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[i][t][r] *= f[r];
-            }
-        }
-        f32x4 d[2][NT];
-        float dwp[NT];  // the scales of the row before
-        auto scale = [&](int i, const f32x4 (&v)[NT], const float (&dw)[NT]) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t], v[t][r], acc[i][t][r]);
-            pin(acc[i]);
+            for (int t = 0; t < HT; ++t) acc[i][h * HT + t] = s[t];
         };
 #pragma unroll
-        for (int u = 0; u < 2 * MT; ++u) {  // tile row u % MT of chunk u / MT
-            const int i = u % MT;
+        for (int v = 0; v < N; ++v) {
+            const int i = v % MT;
             __builtin_amdgcn_sched_barrier(0);
-            if (u == MT / 2) col1 = load_cols(1);
-            if (u + 2 < 2 * MT) row[(u + 2) % 3] = load_row((u + 2) / MT, (u + 2) % MT);
-            if (u == MT) {
+            if (i == 0 && v + MT < N) next = load_cols(buf, (v + MT) / MT / H, (v + MT) / MT % H);
+            const Operands xi = x[i];
+            f32x4 *dv = d[v & 1];
 #pragma unroll
-                for (int t = 0; t < NT; ++t) dwp[t] = col.dw[t];
-                col = col1;
+            for (int t = 0; t < HT; ++t)
+                dv[t] = Q81 ? mfma_h(xi.part[0], col.b[t], f32x4{0.0f, 0.0f, 0.0f, 0.0f})
+                            : mfma(xi.part[0], col.b[t], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+            if constexpr (!Q81) {
+#pragma unroll
+                for (int p = 1; p < 3; ++p)
+#pragma unroll
+                    for (int t = 0; t < HT; ++t) dv[t] = mfma(xi.part[p], col.b[t], dv[t]);
             }
-            const Row &x = row[u % 3];
+            if (v > 0) scale(v - 1);
+            // the next row's operands, if it is the first that uses them; its values two rows on
+            if (v + 1 < N && (v + 1) / MT % H == 0) {
+                const int i1 = (v + 1) % MT;
+                x[i1] = operands(raw[i1]);
+                if ((v + 1) / MT / H == 0) raw[i1] = load_raw(buf, 1, i1);
+            }
+            if (v == 0) raw[0] = load_raw(buf, 1, 0);
 #pragma unroll
-            for (int t = 0; t < NT; ++t) d[u & 1][t] = mfma(x.h, col.b[t], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-#pragma unroll
-            for (int t = 0; t < NT; ++t) d[u & 1][t] = mfma(x.l, col.b[t], d[u & 1][t]);
-            if (u == MT) scale(MT - 1, d[(u - 1) & 1], dwp);
-            else if (u > 0) scale(i - 1, d[(u - 1) & 1], col.dw);
+            for (int t = 0; t < HT; ++t) dwp[t] = col.dw[t];
+            if constexpr (Q81) dxp = xi.dx;
+            if (i == MT - 1) col = next;
         }
-        scale(MT - 1, d[(2 * MT - 1) & 1], col.dw);
+        scale(N - 1);
     };
     // nothing moves across a barrier
     auto sync = [&] {
@@ -456,7 +409,7 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    if (tid < 2) reinterpret_cast<int *>(lds + L::flag)[tid] = -1;
+    if (tid == 0) *again = 0;
     load_w(wr[1], 0);
     load_x(0);
     load_w(wr[0], 1);
@@ -480,18 +433,41 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
         step(wr[0], k);
         if (k + 1 < nstep) step(wr[1], k + 1);
     }
-    if (xlive && xq8 == 0) {
+    if constexpr (!Q81) {
+        __syncthreads();
+        if (*again) {  // uniform, rare: the tile once more, as f32 values
 #pragma unroll
-        for (int p = 0; p < XP; ++p)
-            fbuf(L::inv)[p * (kThreads / 8) + (tid >> 3)] = xs[p].limit > 0.0f ? xs[p].limit * 0x1p-15f : 1.0f;
+            for (int t = 0; t < NT; ++t) {
+                const int o = MODE == kSwiGLU ? o0 + (wn * (NT / 2) + t % (NT / 2)) * 16 + n : o0 + (wn * NT + t) * 16 + n;
+                const uint8_t *wr = (MODE == kSwiGLU && t >= NT / 2 ? a.w1 : a.w0) + static_cast<size_t>(min(o, a.n - 1)) * a.rb;
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    const float *xr = static_cast<const float *>(a.x) +
+                                      static_cast<size_t>(min(m0 + (wm * MT + i) * 16 + n, a.m - 1)) * a.k;
+                    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+                    for (int kb = 0; kb < a.k; kb += 128) {  // (sums of 128 values first: a short chain of roundings)
+                        f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+                        for (int k0 = kb + 8 * g; k0 < min(kb + 128, a.k); k0 += 32) {
+                            Raw8<FMT> r;
+                            raw8<FMT>(wr, k0, r);
+                            float xe[8], v[8];
+                            __builtin_memcpy(xe, __builtin_assume_aligned(xr + k0, 4), sizeof(xe));
+                            values8<FMT>(r, k0, v);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) d = mfma_f32(xe[e], v[e], d);
+                        }
+                        sum += d;
+                    }
+                    acc[i][t] = sum;
+                }
+            }
+        }
     }
-    __syncthreads();
 
     // lane (g, n) holds tokens 4g .. 4g+3 of each 16-token tile, weight row n of each 16-row tile
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const int t0 = (wm * MT + i) * 16 + 4 * g;
-        const f32x4 inv = *reinterpret_cast<const f32x4 *>(fbuf(L::inv) + t0);
 #pragma unroll
         for (int t = 0; t < (MODE == kSwiGLU ? NT / 2 : NT); ++t) {
             const int o = o0 + (wn * (MODE == kSwiGLU ? NT / 2 : NT) + t) * 16 + n;
@@ -499,9 +475,9 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
             for (int r = 0; r < 4; ++r) {
                 if (o >= a.n || m0 + t0 + r >= a.m) continue;
                 float *yp = a.y + static_cast<size_t>(m0 + t0 + r) * a.n + o;
-                const float v = acc[i][t][r] * inv[r];
+                const float v = acc[i][t][r];
                 if constexpr (MODE == kSwiGLU) {
-                    const float u = acc[i][t + NT / 2][r] * inv[r];
+                    const float u = acc[i][t + NT / 2][r];
                     *yp = v / (1.0f + expf(-v)) * u;
                 } else if constexpr (MODE == kAdd) {
                     *yp += v;
@@ -517,39 +493,23 @@ template <int FMT, bool Q81, int MODE, class G>
 hipError_t launch(const GemmArgs &a, hipStream_t s) {
     constexpr int out = MODE == kSwiGLU ? G::BN / 2 : G::BN;
     const dim3 grid = gemm_grid((a.n + out - 1) / out, (a.m + G::BM - 1) / G::BM);
-    hipLaunchKernelGGL((gemm_kernel<FMT, Q81, MODE, G>), grid, dim3(kThreads), Lds<G>::bytes, s, a);
+    hipLaunchKernelGGL((gemm_kernel<FMT, Q81, MODE, G>), grid, dim3(kThreads), (Lds<G, Q81>::bytes), s, a);
     return hipGetLastError();
 }
 
-using Large = Geo<4, 4, 2, 4>;  // 128 tokens x 256 rows
-using Mid = Geo<2, 2, 2, 4>;    // 64 tokens x 128 rows
+// Two and one tiles a row: no register spilled.  Four and two: 20-28 and 0-9 spilled, 223-273 us for [14336, 4096] at
+// 512 tokens against 178-181.
+using Large = Geo<2, 8, 4, 2, 2>;  // 128 tokens x 256 rows
+using Mid = Geo<1, 4, 4, 2, 1>;    // 64 tokens x 128 rows
+static_assert(Large::BM == plan::kGemmLarge.bm && Large::BN == plan::kGemmLarge.bn && Mid::BM == plan::kGemmMid.bm &&
+                  Mid::BN == plan::kGemmMid.bn,
+              "the plan's tiles");
 
-// Microseconds of a launch, measured: a step of a round of workgroups takes 2.5 us with the large tiles
-// (matrix cores, vector ALU and LDS each about half busy); with the middle ones 1.35 us for one workgroup
-// on a CU (a step's latency) and 1.75 us for two, which LDS and registers have room for (Q8_0 [14336, 4096] at
-// 256 tokens 157 us with the large tiles, 117 with two of the middle ones; [28672, 1024] at 128 tokens 47 us
-// with one middle one after the other, 35 with two at a time).  Filling and draining: 12 and 6 us.
-struct GemmPlan {
-    bool large;
-    float us;
-};
-GemmPlan gemm_plan(int n, int k, int m, bool swiglu) {
-    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    const float steps = static_cast<float>((k / 32 + 1) / 2);
-    auto groups = [&](int bm, int bn) {
-        if (swiglu) bn /= 2;
-        return static_cast<int64_t>((n + bn - 1) / bn) * ((m + bm - 1) / bm);
-    };
-    const int64_t lg = groups(Large::BM, Large::BN), mg = groups(Mid::BM, Mid::BN), rest = mg % (2 * cus);
-    const float l = 12.0f + 2.5f * steps * static_cast<float>((lg + cus - 1) / cus);
-    const float d = 6.0f + steps * (1.75f * static_cast<float>(mg / (2 * cus)) +
-                                    (rest == 0 ? 0.0f : rest <= cus ? 1.35f : 1.75f));
-    return l <= d ? GemmPlan{true, l} : GemmPlan{false, d};
-}
+int cu_count() { return device_info().cu_count > 0 ? device_info().cu_count : 256; }
 
 template <int FMT, bool Q81, int MODE>
 hipError_t by_size(const GemmArgs &a, hipStream_t s) {
-    if (gemm_plan(a.n, a.k, a.m, MODE == kSwiGLU).large) return launch<FMT, Q81, MODE, Large>(a, s);
+    if (plan::gemm(FMT, Q81, a.n, a.k, a.m, MODE == kSwiGLU, cu_count()).large) return launch<FMT, Q81, MODE, Large>(a, s);
     return launch<FMT, Q81, MODE, Mid>(a, s);
 }
 
@@ -576,7 +536,9 @@ hipError_t run(int type, const GemmArgs &a, bool q81, int mode, hipStream_t s) {
 
 }  // namespace
 
-float gemm_us(int n, int k, int m, bool swiglu) { return gemm_plan(n, k, m, swiglu).us; }
+float gemm_us(int type, bool q81, int n, int k, int m, bool swiglu) {
+    return plan::gemm(type, q81, n, k, m, swiglu, cu_count()).us;
+}
 
 hipError_t gemm_f32(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const float *x, float *y, int n, int k,
                     int m, int mode, hipStream_t s) {

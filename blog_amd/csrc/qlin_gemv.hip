@@ -90,7 +90,7 @@ hipError_t gemv(int type, const uint8_t *w, size_t rb, const float *x, float *y,
         // the prefill GEMM where its tiles fill the chip or x is long enough to be split once per tile; below
         // that the waves of a workgroup split K (and layouts that kernel does not take run the GEMM too)
         const bool dense = dense_ok(type, w, nullptr, rb, x, k);
-        if (!dense || gemm_us(n, k, m, false) < dense_us(type, n, k, m, false))
+        if (!dense || gemm_us(type, false, n, k, m, false) < dense_us(type, n, k, m, false))
             return gemm_f32(type, w, nullptr, rb, x, y, n, k, m, add, s);
     }
     if (m >= kF32GemmMinRows && f32_gemm_ok(type, w, rb, x, k) &&

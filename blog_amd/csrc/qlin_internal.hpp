@@ -133,11 +133,11 @@ hipError_t dequant(int type, const uint8_t *src, void *out, int64_t n, bool to_f
 
 // Q8_1 activation quantizer (36 B per 32 values) and the weight x Q8_1 matmul.
 hipError_t quantize_q8_1(const float *x, uint8_t *xq, int in_dim, int m, bool raw_sum, hipStream_t s);
-// The prefill GEMM of the 32-block formats (Q4_0, Q5_0, Q8_0) on the fp16 matrix cores (qlin_gemm.hip): f32
-// activations (mode 0: y =, 1: y +=, 2: SwiGLU of the gate rows w0 and the up rows w1) or Q8_1 ones, any
-// layout the entry points accept.  gemm_us, dense_us: the estimated microseconds of gemm_f32 and of
-// dense_matmul (all formats but Q4_K), from which the dispatch chooses.
-float gemm_us(int n, int k, int m, bool swiglu);
+// The prefill GEMM of the 32-block formats (Q4_0, Q5_0, Q8_0) on the matrix cores (qlin_gemm.hip), products exact:
+// f32 activations (mode 0: y =, 1: y +=, 2: SwiGLU of the gate rows w0 and the up rows w1) or Q8_1 ones, any
+// layout the entry points accept.  gemm_us, dense_us: the estimated microseconds of gemm_f32 (q81: gemm_q8_1) and
+// of dense_matmul (all formats but Q4_K), from which the dispatch chooses.
+float gemm_us(int type, bool q81, int n, int k, int m, bool swiglu);
 float dense_us(int type, int n, int k, int m, bool swiglu);
 hipError_t gemm_f32(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, float *y, int n,
                     int k, int m, int mode, hipStream_t s);
@@ -145,7 +145,7 @@ hipError_t gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t
                      hipStream_t s);
 // Q8_0 / Q5_0 / Q4_0 x Q8_1 prefill GEMM on the fp16 matrix cores (qlin_qblk_gemm.hip).
 bool qblk_gemm_ok(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, int in_dim);
-float qblk_gemm_us(int out_dim, int in_dim, int m);  // its estimated microseconds (not Q6_K's)
+float qblk_gemm_us(int type, int out_dim, int in_dim, int m);  // its estimated microseconds (not Q6_K's)
 hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, float *y, int out_dim,
                           int in_dim, int m, hipStream_t s);
 // Q4_K / Q6_K x f32 activations, the prefill GEMM of quant_matmul for m >= kF32GemmMinRows rows, on the

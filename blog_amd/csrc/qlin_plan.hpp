@@ -130,5 +130,52 @@ inline Rows rows(int type, int n, int k, int m, bool swiglu, int cus) {
     return best;
 }
 
+// The prefill GEMM (qlin_gemm.hip): its tiles (bm tokens x bn rows) and the microseconds of a launch, fill + K steps
+// of 64 x the cost of one, fitted as above (4-9% off in the mean): with the large tiles a step per round of
+// workgroups; with the middle ones a step of one workgroup on a CU, or of two at a time, which LDS and registers
+// have room for.
+struct Tile {
+    int bm, bn;
+};
+constexpr Tile kGemmLarge{128, 256}, kGemmMid{64, 128};
+struct Gemm {
+    bool large = false;
+    float us = 0.0f;
+};
+inline Gemm gemm(int type, bool q81, int n, int k, int m, bool swiglu, int cus) {
+    static constexpr struct {
+        float fill, step, mid_fill, mid_two, mid_one;
+    } costs[2][3] = {{{7.3f, 2.5f, 2.8f, 2.08f, 1.41f}, {8.3f, 2.57f, 2.8f, 2.22f, 1.56f}, {7.8f, 2.48f, 2.4f, 1.98f, 1.52f}},
+                     {{7.5f, 1.67f, 1.85f, 1.3f, 0.86f}, {7.6f, 1.71f, 2.6f, 1.41f, 0.99f}, {7.1f, 1.69f, 1.75f, 1.17f, 1.07f}}};
+    const int f = rows_format(type);
+    if (f < 0 || f > 2) return Gemm{};
+    const auto &c = costs[q81 ? 1 : 0][f];
+    const float steps = static_cast<float>((k / 32 + 1) / 2);
+    const int64_t lg = tiles(n, kGemmLarge.bn / (swiglu ? 2 : 1), m, kGemmLarge.bm);
+    const int64_t mg = tiles(n, kGemmMid.bn / (swiglu ? 2 : 1), m, kGemmMid.bm), rest = mg % (2 * cus);
+    const float l = c.fill + c.step * steps * static_cast<float>((lg + cus - 1) / cus);
+    const float d = c.mid_fill + steps * (c.mid_two * static_cast<float>(mg / (2 * cus)) +
+                                          (rest == 0 ? 0.0f : rest <= cus ? c.mid_one : c.mid_two));
+    Gemm g;
+    g.large = l <= d;
+    g.us = g.large ? l : d;
+    return g;
+}
+
+// The Q8_1 GEMM of 64-token tiles (qlin_qblk_gemm.hip), for the 32-block formats: the default tiles, the small ones
+// where those would leave more than half the CUs idle, and the microseconds of a launch, fill + units of 256
+// values x the cost of one per round of workgroups, fitted as above (4-9% off).
+constexpr Tile kQblkLarge{64, 256}, kQblkSmall{32, 128};
+inline bool qblk_small(int n, int m, int cus) { return tiles(n, kQblkLarge.bn, m, kQblkLarge.bm) * 2 < cus; }
+inline float qblk_us(int type, int n, int k, int m, int cus) {
+    static constexpr float fill[3] = {3.9f, 3.75f, 4.15f}, small[3] = {2.89f, 3.03f, 2.97f}, large[3] = {6.8f, 6.65f, 6.55f};
+    const int f = rows_format(type);
+    if (f < 0 || f > 2) return 0.0f;
+    const bool s = qblk_small(n, m, cus);
+    const Tile t = s ? kQblkSmall : kQblkLarge;
+    return fill[f] + static_cast<float>((tiles(n, t.bn, m, t.bm) + cus - 1) / cus) * (s ? small[f] : large[f]) *
+                         static_cast<float>((k + 255) / 256);
+}
+
 }  // namespace plan
 }  // namespace qlin

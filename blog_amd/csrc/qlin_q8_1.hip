@@ -55,12 +55,11 @@ hipError_t matmul_q8_1(int type, const uint8_t *w, size_t rb, const uint8_t *xq,
     if (waves == 0) return hipSuccess;
     if (type == T_Q4_K && q4k_gemm_ok(w, rb, xq, in_dim)) return q4k_gemm_q8_1(w, rb, xq, y, out_dim, in_dim, m, s);
     if (type == T_Q4_0 || type == T_Q5_0 || type == T_Q8_0) {
-        // the prefill GEMM shared with f32 activations where its 128 x 256 tiles win (from about two rounds
-        // of the 64 x 256 ones: Q8_0 [14336, 4096] at 512 tokens 315 -> 165 us, Q5_0 [2048, 1408] 28.7 against
-        // 34 us), and for layouts the other does not take
+        // the prefill GEMM shared with f32 activations where the estimates have it the faster one (Q8_0
+        // [14336, 4096] at 512 tokens 303 -> 121 us), and for layouts the other does not take
         const bool ok = qblk_gemm_ok(type, w, rb, xq, in_dim);
         if ((reinterpret_cast<uintptr_t>(xq) & 3u) == 0 &&
-            (ok ? gemm_us(out_dim, in_dim, m, false) < qblk_gemm_us(out_dim, in_dim, m) : m > 1))
+            (ok ? gemm_us(type, true, out_dim, in_dim, m, false) < qblk_gemm_us(type, out_dim, in_dim, m) : m > 1))
             return gemm_q8_1(type, w, rb, xq, y, out_dim, in_dim, m, s);
     }
     if (qblk_gemm_ok(type, w, rb, xq, in_dim)) return qblk_gemm_q8_1(type, w, rb, xq, y, out_dim, in_dim, m, s);

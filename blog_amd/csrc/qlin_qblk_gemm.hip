@@ -27,6 +27,7 @@
 // last block of a row is odd); an odd block's start at most 2 bytes before it.
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
+#include "qlin_plan.hpp"
 
 #include <type_traits>
 
@@ -614,20 +615,12 @@ bool qblk_gemm_ok(int type, const uint8_t *w, size_t rb, const uint8_t *xq, int 
            (reinterpret_cast<uintptr_t>(xq) & 3u) == 0;
 }
 
-// Measured: a round of workgroups takes about 9.8 us per unit of 256 values on the default tiles, 4.7 on
-// the small ones (the 32-block formats').
-static bool small_tiles(int out_dim, int m) {
-    const int64_t large = static_cast<int64_t>((out_dim + GeoLarge::kBN - 1) / GeoLarge::kBN) *
-                          ((m + GeoLarge::kBM - 1) / GeoLarge::kBM);
-    return QLIN_QBLK_SMALL && large * 2 < device_info().cu_count;
-}
-float qblk_gemm_us(int out_dim, int in_dim, int m) {
-    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    const bool small = small_tiles(out_dim, m);
-    const int bn = small ? GeoSmall::kBN : GeoLarge::kBN, bm = small ? GeoSmall::kBM : GeoLarge::kBM;
-    const int64_t wgs = static_cast<int64_t>((out_dim + bn - 1) / bn) * ((m + bm - 1) / bm);
-    return 3.0f + static_cast<float>((wgs + cus - 1) / cus) * (small ? 4.7f : 9.8f) * static_cast<float>((in_dim + 255) / 256);
-}
+static_assert(GeoLarge::kBM == plan::kQblkLarge.bm && GeoLarge::kBN == plan::kQblkLarge.bn &&
+                  GeoSmall::kBM == plan::kQblkSmall.bm && GeoSmall::kBN == plan::kQblkSmall.bn,
+              "the plan's tiles");
+static int cu_count() { return device_info().cu_count > 0 ? device_info().cu_count : 256; }
+static bool small_tiles(int out_dim, int m) { return QLIN_QBLK_SMALL && plan::qblk_small(out_dim, m, cu_count()); }
+float qblk_gemm_us(int type, int out_dim, int in_dim, int m) { return plan::qblk_us(type, out_dim, in_dim, m, cu_count()); }
 
 hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t rb, const uint8_t *xq, float *y, int out_dim,
                           int in_dim, int m, hipStream_t s) {

@@ -579,8 +579,9 @@ def test_rows_of_f32(qtype, N, K, m, mode):
 
 @pytest.mark.parametrize("qtype,N,m", [(Q8_0, 300, 70), (Q6_K, 300, 40), (Q4_0, 8300, 130)])
 def test_rows_of_f32_token_scales(qtype, N, m):
-    """Tokens of very different magnitudes, one whose large values come last or first (the scale changes on
-    the way), zeros, and an infinite or NaN value, which reaches its own token's outputs alone."""
+    """Tokens of very different magnitudes, one whose large values come last or first, zeros, and an infinite
+    or NaN value, which reaches its own token's outputs alone; each output within the bound of its own
+    sum |w||x|."""
     K = 1024
     w, rb, vals = qgen.random_matrix(qtype, N, K, seed=195)
     rng = np.random.default_rng(196)
@@ -602,7 +603,7 @@ def test_rows_of_f32_token_scales(qtype, N, m):
     fine = np.r_[0:15, 18:m]
     ref = orc.matmul_f64(qtype, w, rb, x[fine], N, K)
     scale = np.abs(x[fine].astype(np.float64)) @ np.abs(vals.astype(np.float64)).T
-    err = np.abs(got[fine] - ref) / np.maximum(scale.max(axis=1, keepdims=True), 1e-300)
+    err = np.abs(got[fine] - ref) / np.maximum(scale, 1e-300)
     assert np.isfinite(got[fine]).all() and err.max() <= COND, float(err.max())
     assert not got[10].any()
     for t, k in ((15, 77), (16, 900)):           # w inf: infinite with the weight's sign, NaN for a zero weight
@@ -631,7 +632,8 @@ def _zero_weight(qtype, w, rb, vals, rows, k):
     vals[rows, k] = 0.0
 
 
-WIDE_ROWS = [(Q8_0, 300, 70), (Q6_K, 300, 40), (Q5_0, 300, 20), (Q4_0, 300, 9)]
+WIDE_ROWS = [(Q8_0, 300, 70), (Q6_K, 300, 40), (Q5_0, 300, 20), (Q4_0, 300, 9),
+             (Q4_0, 8300, 130), (Q5_0, 14400, 260), (Q8_0, 14400, 260)]   # the prefill GEMM's tiles
 
 
 @pytest.mark.parametrize("qtype,N,m", WIDE_ROWS)
@@ -660,10 +662,11 @@ def test_rows_of_f32_over_the_whole_range(qtype, N, m):
     yd = empty_f32(m, N)
     qlin.quant_matmul(qtype, dev(w), rb, dev(x), yd, N, K, m)
     got = host(yd)
-    fine = np.r_[0:6, 7:m]
+    fine = np.r_[0:6, 7, m - 1]
     ref = orc.matmul_f64(qtype, w, rb, x[fine], N, K)
     scale = np.abs(x[fine].astype(np.float64)) @ np.abs(vals.astype(np.float64)).T
     err = np.abs(got[fine] - ref) / scale
+    assert np.isfinite(got[7:]).all()
     assert np.isfinite(got[fine]).all() and err.max() <= COND, (err.max(axis=1), np.isfinite(got[fine]).all(axis=1))
     w0 = vals[:, k0].astype(np.float64)
     assert np.isnan(got[6][w0 == 0]).all()
@@ -686,6 +689,28 @@ def test_matmul_q8_1_shared_gemm(qtype, N, K, m):
     ref = orc.matmul_q8_1(qtype, w, rb, np.ascontiguousarray(xq.reshape(m, rbx)[toks]).reshape(-1), N, K, toks.size)
     assert np.isfinite(host(yd)).all()
     assert normwise_rel_err(host(yd)[toks], ref) <= FP32
+
+
+@pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 14400, 1024, 260), (Q4_0, 14400, 1056, 66)])
+def test_matmul_q8_1_shared_gemm_block_scales(qtype, N, K, m):
+    """A Q8_1 token whose blocks' scales differ by 1e9, with weight 0 under the large block in every second
+    row: a block's dot is an exact integer whatever the others' scales are."""
+    w, rb, vals = qgen.random_matrix(qtype, N, K, seed=395)
+    bb = qgen.BLOCK[qtype][1]
+    w.reshape(N, rb)[::2, bb:bb + 2] = 0          # d of block 1
+    vals[::2, 32:64] = 0.0
+    x = qgen.random_x(m, K, seed=396) * np.float32(1e-2)
+    x[:, 32:64] *= np.float32(2e8)
+    xq = orc.quantize_q8_1(x.reshape(-1), m * K)
+    banner(f"q8_1 shared gemm block scales type={qtype} {m}x{K}x{N}")
+    yd = empty_f32(m, N)
+    qlin.quant_matmul_q8_1(qtype, dev(w), rb, dev(xq), yd, N, K, m)
+    toks = np.unique(np.r_[0, m // 2, m - 1])
+    rbx = orc.q8_1_row_bytes(K)
+    ref = orc.matmul_q8_1(qtype, w, rb, np.ascontiguousarray(xq.reshape(m, rbx)[toks]).reshape(-1), N, K, toks.size)
+    scale = np.abs(x[toks].astype(np.float64)) @ np.abs(vals.astype(np.float64)).T
+    err = np.abs(host(yd)[toks] - ref) / scale
+    assert err.max() <= COND, float(err.max())
 
 
 # ---- MoE ----------------------------------------------------------------------------------------
