@@ -145,7 +145,6 @@ hipError_t gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t
                      hipStream_t s);
 // Q8_0 / Q5_0 / Q4_0 x Q8_1 prefill GEMM on the fp16 matrix cores (qlin_qblk_gemm.hip).
 bool qblk_gemm_ok(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, int in_dim);
-float qblk_gemm_us(int type, int out_dim, int in_dim, int m);  // its estimated microseconds (not Q6_K's)
 hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, float *y, int out_dim,
                           int in_dim, int m, hipStream_t s);
 // Q4_K / Q6_K x f32 activations, the prefill GEMM of quant_matmul for m >= kF32GemmMinRows rows, on the

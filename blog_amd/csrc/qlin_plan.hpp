@@ -177,5 +177,23 @@ inline float qblk_us(int type, int n, int k, int m, int cus) {
                          static_cast<float>((k + 255) / 256);
 }
 
+// The block dots of matmul_q8_1_kernel (qlin_q8_1.hip, any layout): a wave per output, 64 blocks of K at a time.
+// Measured per output and 64 blocks: Q8_0 [512, 18976] at 64 rows 117 us, [2048, 352] at 8 rows 7.9.
+inline float block_dots_us(int type, int n, int k, int m) {
+    static constexpr float dot[3] = {3.75e-4f, 4.3e-4f, 3.5e-4f};
+    const int f = rows_format(type);
+    const float rounds = static_cast<float>((k / 32 + 63) / 64);
+    return 2.0f + rounds * (0.3f + dot[f < 0 || f > 2 ? 1 : f] * static_cast<float>(m) * static_cast<float>(n));
+}
+// The kernel of a 32-block product with Q8_1 activations: the cheaper GEMM where the 64-token one takes the layout
+// (qblk_ok), else the other GEMM against the block dots (Q8_0 [512, 18976] at 2 rows: 270 us against 9.7; from 16
+// rows of [4096, 4128] on the GEMM).
+enum class Q81 { kGemm, kQblk, kBlockDots };
+inline Q81 q8_1_route(int type, int n, int k, int m, bool qblk_ok, bool gemm_ok, int cus) {
+    const float other = qblk_ok ? qblk_us(type, n, k, m, cus) : block_dots_us(type, n, k, m);
+    if (gemm_ok && gemm(type, true, n, k, m, false, cus).us < other) return Q81::kGemm;
+    return qblk_ok ? Q81::kQblk : Q81::kBlockDots;
+}
+
 }  // namespace plan
 }  // namespace qlin

@@ -2,6 +2,7 @@
 // The block quantizer and the per-type block dots (kernel.cu:1679-1720, 2305-2402) are in qlin_q8_1.hpp.
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
+#include "qlin_plan.hpp"
 #include "qlin_q8_1.hpp"
 
 namespace qlin {
@@ -55,12 +56,10 @@ hipError_t matmul_q8_1(int type, const uint8_t *w, size_t rb, const uint8_t *xq,
     if (waves == 0) return hipSuccess;
     if (type == T_Q4_K && q4k_gemm_ok(w, rb, xq, in_dim)) return q4k_gemm_q8_1(w, rb, xq, y, out_dim, in_dim, m, s);
     if (type == T_Q4_0 || type == T_Q5_0 || type == T_Q8_0) {
-        // the prefill GEMM shared with f32 activations where the estimates have it the faster one (Q8_0
-        // [14336, 4096] at 512 tokens 303 -> 121 us), and for layouts the other does not take
-        const bool ok = qblk_gemm_ok(type, w, rb, xq, in_dim);
-        if ((reinterpret_cast<uintptr_t>(xq) & 3u) == 0 &&
-            (ok ? gemm_us(type, true, out_dim, in_dim, m, false) < qblk_gemm_us(type, out_dim, in_dim, m) : m > 1))
-            return gemm_q8_1(type, w, rb, xq, y, out_dim, in_dim, m, s);
+        const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+        const plan::Q81 route = plan::q8_1_route(type, out_dim, in_dim, m, qblk_gemm_ok(type, w, rb, xq, in_dim),
+                                                 (reinterpret_cast<uintptr_t>(xq) & 3u) == 0, cus);
+        if (route == plan::Q81::kGemm) return gemm_q8_1(type, w, rb, xq, y, out_dim, in_dim, m, s);
     }
     if (qblk_gemm_ok(type, w, rb, xq, in_dim)) return qblk_gemm_q8_1(type, w, rb, xq, y, out_dim, in_dim, m, s);
     const dim3 grid(static_cast<unsigned>((waves + 3) / 4));

@@ -79,6 +79,17 @@ int main() {
         CHECK(!c.ok);
         CHECK(!stream(q4k, true, 16, 256, 64, 6, 256, kMaxLds, kMaxLds).ok);  // unreadable kernels
     }
+    // Q8_1 products in layouts that the 64-token GEMM does not take: few outputs stay with the block dots,
+    // however long their rows; enough of them take the other GEMM.  (Q4_0 2, Q5_0 6, Q8_0 8)
+    for (int type : {2, 6, 8}) {
+        for (int m : {1, 2, 8, 64}) CHECK(q8_1_route(type, 512, 18976, m, false, true, 256) == Q81::kBlockDots);
+        CHECK(q8_1_route(type, 300, 1056, 66, false, true, 256) == Q81::kBlockDots);
+        CHECK(q8_1_route(type, 64, 96, 2, false, true, 256) == Q81::kBlockDots);
+        CHECK(q8_1_route(type, 14336, 4128, 64, false, true, 256) == Q81::kGemm);
+        CHECK(q8_1_route(type, 14336, 4128, 64, false, false, 256) == Q81::kBlockDots);  // 2-byte aligned activations
+        CHECK(q8_1_route(type, 14336, 4096, 512, true, true, 256) == Q81::kGemm);
+        CHECK(q8_1_route(type, 14336, 4096, 8, true, true, 256) == Q81::kQblk);
+    }
     std::printf("%s: %ld gemv plans accepted, %ld refused\n", failures ? "FAILED" : "ok", accepted, refused);
     return failures ? 1 : 0;
 }
