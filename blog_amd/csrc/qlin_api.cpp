@@ -312,10 +312,10 @@ int qlin_launch_quant_swiglu_rows(int type, const uint8_t *wg, const uint8_t *wu
     if ((rc = check_f32(x, work)) || (rc = check_f32(act, work))) return rc;
     if (!work) return QLIN_OK;
     if (m > 1 && g_rb == u_rb && (type == QLIN_TYPE_Q4_0 || type == QLIN_TYPE_Q5_0 || type == QLIN_TYPE_Q8_0) &&
-        (!qlin::dense_ok(type, wg, wu, g_rb, x, in_dim) ||
+        (!qlin::dense_ok(type, wg, wu, g_rb, x, ffn_dim, in_dim) ||
          qlin::gemm_us(type, false, ffn_dim, in_dim, m, true) < qlin::dense_us(type, ffn_dim, in_dim, m, true)))
         return launched(qlin::gemm_f32(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));
-    if (m > 1 && g_rb == u_rb && qlin::dense_ok(type, wg, wu, g_rb, x, in_dim))
+    if (m > 1 && g_rb == u_rb && qlin::dense_ok(type, wg, wu, g_rb, x, ffn_dim, in_dim))
         return launched(qlin::dense_matmul(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));
     for (int r = 0; r < m; ++r) {
         const hipError_t e = qlin::swiglu(type, wg, wu, g_rb, u_rb, x + static_cast<size_t>(r) * in_dim,
@@ -954,7 +954,7 @@ int qlin_moe_ffn_decode_grouped_logits(int gu_type, const uint8_t *gate, const u
     const size_t g_rb = g_eb / static_cast<size_t>(ffn_dim);
     const bool fuse = k > 0 && shared && tokens > 1 &&
                       qlin::moe_grouped_up_ok(gu_type, gate, up, g_eb, g_rb, x, in_dim, ffn_dim, n_experts, tokens * k) &&
-                      qlin::dense_ok(shared_type, shared_down, nullptr, shared_down_rb, sact, shared_ffn);
+                      qlin::dense_ok(shared_type, shared_down, nullptr, shared_down_rb, sact, hidden, shared_ffn);
     if (fuse) {
         const size_t d_eb = down_bytes / static_cast<size_t>(n_experts);
         const size_t d_rb = d_eb / static_cast<size_t>(hidden);
@@ -964,7 +964,7 @@ int qlin_moe_ffn_decode_grouped_logits(int gu_type, const uint8_t *gate, const u
         bool shared_done = false;
         const qlin::SharedUp sh{shared_gate, shared_up, shared_gate_up_rb, sact, shared_ffn, &shared_done};
         const bool sh_ok = shared_type == QLIN_TYPE_Q4_K && in_dim % 256 == 0 &&
-                           qlin::dense_ok(shared_type, shared_gate, shared_up, shared_gate_up_rb, x, in_dim);
+                           qlin::dense_ok(shared_type, shared_gate, shared_up, shared_gate_up_rb, x, shared_ffn, in_dim);
         hipError_t e = qlin::moe_grouped(gu_type, gate, up, g_eb, g_rb, down_type, down, d_eb, d_rb, n_experts, ffn_dim,
                                          in_dim, hidden, x, nullptr, nullptr, workspace, out, tokens, k, stream(),
                                          &router, &routed, sh_ok ? &sh : nullptr);

@@ -363,7 +363,7 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
         const int c = min(8 * kUnit * u + lc, 8 * nblk - 8 + (lc & 7));
 #pragma unroll
         for (int p = 0; p < 2 * kUnit; ++p)
-            x[p] = reinterpret_cast<const f32x4 *>(a.x + static_cast<size_t>(min(t0 + 16 * i + 2 * p + lt, a.m - 1)) * K)[c];
+            __builtin_memcpy(&x[p], __builtin_assume_aligned(a.x + static_cast<size_t>(min(t0 + 16 * i + 2 * p + lt, a.m - 1)) * K + 4 * c, 4), 16);
     };
     auto turn_x = [&](const f32x4 (&x)[2 * kUnit], f32x4 (&r)[2 * kUnit]) {
 #pragma unroll
@@ -540,12 +540,10 @@ hipError_t launch_dense(const DenseArgs &a, int mode, hipStream_t s) {
 
 }  // namespace
 
-bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const float *x, int k) {
-    const auto al = [](const void *p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & (m - 1)) == 0; };
-    if (type == T_Q4_K) return k % 256 == 0 && rb % 16 == 0 && al(w0, 16) && (!w1 || al(w1, 16)) && al(x, 16);
-    if (type != T_Q4_0 && type != T_Q5_0 && type != T_Q8_0 && type != T_Q6_K) return false;
-    // blocks are read at their 2-byte alignment
-    return k % 32 == 0 && rb % 2 == 0 && al(w0, 2) && (!w1 || al(w1, 2)) && al(x, 16);
+bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const float *x, int n, int k) {
+    const auto at = [](const void *p) { return reinterpret_cast<uintptr_t>(p); };
+    if (type == T_Q4_K) return k % 256 == 0 && rb % 16 == 0 && (at(w0) | at(w1) | at(x)) % 16 == 0;
+    return plan::rows_layout_ok(type, at(w0), at(w1), rb, at(x), n, k);
 }
 
 float dense_us(int type, int n, int k, int m, bool swiglu) { return plan::rows(type, n, k, m, swiglu, cu_count()).us; }

@@ -87,16 +87,16 @@ hipError_t gemv(int type, const uint8_t *w, size_t rb, const float *x, float *y,
     if (type == T_Q4_K && m == 1 && q4k_stream_ok(&w, 1, rb, x, n, k, false))
         return q4k_stream_gemv(&w, &y, &n, 1, rb, x, k, add, s);
     if (m > 1 && (type == T_Q4_0 || type == T_Q5_0 || type == T_Q8_0)) {
-        // the prefill GEMM where its tiles fill the chip or x is long enough to be split once per tile; below
-        // that the waves of a workgroup split K (and layouts that kernel does not take run the GEMM too)
-        const bool dense = dense_ok(type, w, nullptr, rb, x, k);
+        // the prefill GEMM where its tiles fill the chip or x is long enough to be staged once per tile; below
+        // that the waves of a workgroup split K (rows_kernel takes every layout that gets here)
+        const bool dense = dense_ok(type, w, nullptr, rb, x, n, k);
         if (!dense || gemm_us(type, false, n, k, m, false) < dense_us(type, n, k, m, false))
             return gemm_f32(type, w, nullptr, rb, x, y, n, k, m, add, s);
     }
     if (m >= kF32GemmMinRows && f32_gemm_ok(type, w, rb, x, k) &&
-        (type != T_Q6_K || !dense_ok(type, w, nullptr, rb, x, k) || f32_gemm_us_q6k(n, k, m) <= dense_us(type, n, k, m, false)))
+        (type != T_Q6_K || !dense_ok(type, w, nullptr, rb, x, n, k) || f32_gemm_us_q6k(n, k, m) <= dense_us(type, n, k, m, false)))
         return f32_gemm(type, w, rb, x, y, n, k, m, add, s);
-    if (m > 1 && dense_ok(type, w, nullptr, rb, x, k)) return dense_matmul(type, w, nullptr, rb, x, y, n, k, m, add, s);
+    if (m > 1 && dense_ok(type, w, nullptr, rb, x, n, k)) return dense_matmul(type, w, nullptr, rb, x, y, n, k, m, add, s);
     return gemv_generic(type, w, rb, x, y, n, k, m, add, s);
 }
 

@@ -97,7 +97,7 @@ hipError_t mfma_down_routed(int type, const uint8_t *wd, size_t expert_bytes, si
 // to about 2^-17 of itself), the other formats with all of x in three bf16 parts.
 // Mode 0 stores y[r, o], 1 adds into it, 2 writes act[r, o] = silu(gate . x_r) * (up . x_r) with w1 the up
 // matrix.
-bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, int in_dim);
+bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, int out_dim, int in_dim);
 // mode 1 (y +=) with combine: y = (y + the routed total) + the product, as the combine launch and then
 // the plain mode 1 give it
 hipError_t dense_matmul(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, float *y,

@@ -98,7 +98,7 @@ inline int64_t tiles(int n, int bn, int m, int bm) {
 // of 16 per workgroup, one workgroup on a CU at a time, whose 8 waves take units of 128 values of K in turn.
 // us is `base` plus, per round of workgroups, round + unit x (units of a wave): least squares of the logarithm over
 // the tiles of 36 shapes of each format (n 512 .. 32768, k 512 .. 16384, m 2 .. 700), 9-10% off in the mean; the
-// kernel it picks is 0.2% slower in the mean than the fastest, 13% at most.  Larger tiles split x and read the
+// kernel it picks is at most 0.4% slower in the mean than the fastest, and 13% at one shape.  Larger tiles split x and read the
 // weights for more products, smaller ones fill the chip.  Q6_K has no 2 x 4 tiles (they spill: 8.0 us a unit, as
 // much per product as 2 x 3's 5.7).
 struct Rows {
@@ -111,7 +111,7 @@ inline Rows rows(int type, int n, int k, int m, bool swiglu, int cus) {
         float base, round[6], unit[6];
     } costs[4] = {{0.75f, {0.95f, 1.55f, 1.4f, 2.4f, 3.1f, 3.3f}, {1.45f, 1.98f, 2.42f, 3.1f, 4.1f, 5.2f}},
                   {0.8f, {0.9f, 1.6f, 1.55f, 2.3f, 2.9f, 3.6f}, {1.63f, 2.31f, 2.58f, 3.5f, 4.6f, 5.6f}},
-                  {1.7f, {0.9f, 1.1f, 1.15f, 1.85f, 2.2f, 2.85f}, {1.53f, 2.39f, 2.62f, 3.5f, 4.5f, 5.7f}},
+                  {0.8f, {1.2f, 1.5f, 1.35f, 2.2f, 2.7f, 3.55f}, {1.55f, 2.41f, 2.64f, 3.5f, 4.5f, 5.6f}},
                   {1.45f, {0.95f, 1.15f, 1.25f, 1.4f, 2.45f, 0.0f}, {1.83f, 3.2f, 2.86f, 4.55f, 5.7f, 0.0f}}};
     const int f = rows_format(type);
     Rows best;
@@ -193,6 +193,13 @@ inline Q81 q8_1_route(int type, int n, int k, int m, bool qblk_ok, bool gemm_ok,
     const float other = qblk_ok ? qblk_us(type, n, k, m, cus) : block_dots_us(type, n, k, m);
     if (gemm_ok && gemm(type, true, n, k, m, false, cus).us < other) return Q81::kGemm;
     return qblk_ok ? Q81::kQblk : Q81::kBlockDots;
+}
+
+// The layouts that rows_kernel reads: blocks at 2-byte and x at 4-byte alignment (a 16-byte load on a dword
+// boundary runs as an aligned one), a lone row at any stride.
+inline bool rows_layout_ok(int type, uintptr_t w0, uintptr_t w1, size_t row_bytes, uintptr_t x, int n, int k) {
+    return rows_format(type) >= 0 && k % (type == 14 ? 256 : 32) == 0 && (n <= 1 || row_bytes % 2 == 0) && w0 % 2 == 0 &&
+           w1 % 2 == 0 && x % 4 == 0;
 }
 
 }  // namespace plan

@@ -90,6 +90,18 @@ int main() {
         CHECK(q8_1_route(type, 14336, 4096, 512, true, true, 256) == Q81::kGemm);
         CHECK(q8_1_route(type, 14336, 4096, 8, true, true, 256) == Q81::kQblk);
     }
+    // the smallest products stay with rows_kernel (2.5 us for [16, 32] at 2 rows; the GEMM takes 3.7)
+    for (int type : {2, 6, 8})
+        CHECK(rows(type, 16, 32, 2, false, 256).us < gemm(type, false, 16, 32, 2, false, 256).us);
+    // rows_kernel takes what the entry points accept: x on any float, blocks on any 2 bytes, a lone row at an odd
+    // stride (Q6_K 14; Q4_K 12 has a kernel of its own)
+    for (int type : {2, 6, 8, 14}) {
+        for (uintptr_t x : {0, 4, 8, 12}) CHECK(rows_layout_ok(type, 2, 6, 210, 64 + x, 100, 256));
+        CHECK(rows_layout_ok(type, 16, 0, 211, 64, 1, 256));
+        CHECK(!rows_layout_ok(type, 16, 0, 211, 64, 2, 256));
+        CHECK(!rows_layout_ok(type, 16, 0, 210, 66, 100, 256));
+    }
+    CHECK(!rows_layout_ok(12, 16, 0, 144, 64, 100, 256));
     std::printf("%s: %ld gemv plans accepted, %ld refused\n", failures ? "FAILED" : "ok", accepted, refused);
     return failures ? 1 : 0;
 }

@@ -613,6 +613,32 @@ def test_rows_of_f32_token_scales(qtype, N, m):
     assert np.isnan(got[17]).all()
 
 
+@pytest.mark.parametrize("mode", ["store", "add", "swiglu"])
+@pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 100, 96, 5), (Q5_0, 33, 1056, 17), (Q4_0, 520, 160, 40), (Q6_K, 70, 512, 3),
+                                         (Q8_0, 1, 256, 6), (Q4_K, 70, 512, 3)])
+def test_rows_of_f32_off_16_bytes(qtype, N, K, m, mode):
+    """Activations that begin on a float but not on 16 bytes, and a lone row at an odd stride."""
+    w, rb, vals = qgen.random_matrix(qtype, N, K, seed=K + m)
+    w2, _, _ = qgen.random_matrix(qtype, N, K, seed=K + m + 1)
+    x = qgen.random_x(m, K, seed=N + m)
+    stride = rb + 1 if N == 1 else rb
+    banner(f"rows off 16 bytes type={qtype} {m}x{K}x{N} {mode}")
+    ref = orc.matmul_f64(qtype, w, rb, x, N, K)
+    for shift in (1, 3):
+        xd = torch.cat([torch.zeros(shift, device="cuda"), dev(x).view(-1)])[shift:]
+        assert xd.data_ptr() % 16
+        yd = torch.zeros(m, N, device="cuda")
+        if mode == "swiglu":
+            qlin.quant_swiglu_rows(qtype, dev(w), dev(w2), stride, stride, xd, yd, N, K, m)
+            u = orc.matmul_f64(qtype, w2, rb, x, N, K)
+            with np.errstate(over="ignore"):
+                want = ref / (1.0 + np.exp(-ref)) * u
+            assert normwise_rel_err(host(yd), want) <= 2 * FP32
+        else:
+            (qlin.quant_matmul_add if mode == "add" else qlin.quant_matmul)(qtype, dev(w), stride, xd, yd, N, K, m)
+            assert normwise_rel_err(host(yd), ref) <= FP32
+
+
 def _zero_weight(qtype, w, rb, vals, rows, k):
     """Sets element k (k % 32 < 16; Q6_K: 64 <= k < 80) of the rows to weight 0."""
     b = w.reshape(-1, rb)
