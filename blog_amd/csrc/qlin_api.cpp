@@ -311,12 +311,14 @@ int qlin_launch_quant_swiglu_rows(int type, const uint8_t *wg, const uint8_t *wu
     const bool work = ffn_dim > 0 && m > 0;
     if ((rc = check_f32(x, work)) || (rc = check_f32(act, work))) return rc;
     if (!work) return QLIN_OK;
-    if (m > 1 && g_rb == u_rb && (type == QLIN_TYPE_Q4_0 || type == QLIN_TYPE_Q5_0 || type == QLIN_TYPE_Q8_0) &&
-        (!qlin::dense_ok(type, wg, wu, g_rb, x, ffn_dim, in_dim) ||
-         qlin::gemm_us(type, false, ffn_dim, in_dim, m, true) < qlin::dense_us(type, ffn_dim, in_dim, m, true)))
-        return launched(qlin::gemm_f32(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));
-    if (m > 1 && g_rb == u_rb && qlin::dense_ok(type, wg, wu, g_rb, x, ffn_dim, in_dim))
-        return launched(qlin::dense_matmul(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));
+    if (m > 1 && g_rb == u_rb) {
+        const qlin::plan::Product kernel = qlin::plan::swiglu_product(
+            type, ffn_dim, in_dim, m, qlin::dense_ok(type, wg, wu, g_rb, x, ffn_dim, in_dim), qlin::cu_count());
+        if (kernel == qlin::plan::Product::kGemm)
+            return launched(qlin::gemm_f32(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));
+        if (kernel == qlin::plan::Product::kDense)
+            return launched(qlin::dense_matmul(type, wg, wu, g_rb, x, act, ffn_dim, in_dim, m, 2, stream()));
+    }
     for (int r = 0; r < m; ++r) {
         const hipError_t e = qlin::swiglu(type, wg, wu, g_rb, u_rb, x + static_cast<size_t>(r) * in_dim,
                                           act + static_cast<size_t>(r) * ffn_dim, ffn_dim, in_dim, stream());
@@ -918,8 +920,8 @@ size_t qlin_moe_ffn_workspace_bytes(int tokens, int k, int n_experts, int ffn_di
 
 // MoE::forward's routed and shared experts (MoE.cpp:29-52, after the norm, before the residual add):
 // the batched routed decode from the logits, then the shared experts' SwiGLU and down-add.  When the
-// shared down-add takes the m > 1 matrix-core kernel, that launch also applies the routed combine
-// (one launch fewer); either way out gets (out + routed) + shared, as the three calls give it.
+// shared down-add's own call would take dense_matmul, that launch also applies the routed combine (one
+// launch fewer); either way out gets (out + routed) + shared, as the three calls give it, bit for bit.
 int qlin_moe_ffn_decode_grouped_logits(int gu_type, const uint8_t *gate, const uint8_t *up, size_t gate_up_bytes,
                                        int down_type, const uint8_t *down, size_t down_bytes, int n_experts,
                                        int ffn_dim, int in_dim, int hidden, int shared_type, const uint8_t *shared_gate,
@@ -954,7 +956,8 @@ int qlin_moe_ffn_decode_grouped_logits(int gu_type, const uint8_t *gate, const u
     const size_t g_rb = g_eb / static_cast<size_t>(ffn_dim);
     const bool fuse = k > 0 && shared && tokens > 1 &&
                       qlin::moe_grouped_up_ok(gu_type, gate, up, g_eb, g_rb, x, in_dim, ffn_dim, n_experts, tokens * k) &&
-                      qlin::dense_ok(shared_type, shared_down, nullptr, shared_down_rb, sact, hidden, shared_ffn);
+                      qlin::rows_product(shared_type, shared_down, shared_down_rb, sact, hidden, shared_ffn, tokens) ==
+                          qlin::plan::Product::kDense;
     if (fuse) {
         const size_t d_eb = down_bytes / static_cast<size_t>(n_experts);
         const size_t d_rb = d_eb / static_cast<size_t>(hidden);

@@ -510,13 +510,14 @@ hipError_t launch_rows(const DenseArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-int cu_count() { return device_info().cu_count > 0 ? device_info().cu_count : 256; }
-
 template <int T, int MODE>
 hipError_t by_shape(const DenseArgs &a, hipStream_t s) {
     const plan::Rows p = plan::rows(T, a.n, a.k, a.m, MODE == kSwiGLU, cu_count());
     if constexpr (MODE != kSwiGLU) {
-        if (p.nt == 1) return p.tt == 1 ? launch_rows<T, MODE, 1, 1>(a, s) : launch_rows<T, MODE, 1, 2>(a, s);
+        if constexpr (T == T_Q6_K) {
+            if (p.nt == 1 && p.tt == 2) return launch_rows<T, MODE, 1, 2>(a, s);
+        }
+        if (p.nt == 1) return launch_rows<T, MODE, 1, 1>(a, s);
     }
     if constexpr (T != T_Q6_K) {
         if (p.tt == 4) return launch_rows<T, MODE, 2, 4>(a, s);
@@ -545,8 +546,6 @@ bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const f
     if (type == T_Q4_K) return k % 256 == 0 && rb % 16 == 0 && (at(w0) | at(w1) | at(x)) % 16 == 0;
     return plan::rows_layout_ok(type, at(w0), at(w1), rb, at(x), n, k);
 }
-
-float dense_us(int type, int n, int k, int m, bool swiglu) { return plan::rows(type, n, k, m, swiglu, cu_count()).us; }
 
 hipError_t dense_matmul(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const float *x, float *y, int n,
                         int k, int m, int mode, hipStream_t s, const RouteCombine *combine) {

@@ -27,6 +27,7 @@
 // register set reloaded part by part with the next super-block as in the Q8_1 GEMM.
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
+#include "qlin_plan.hpp"
 
 #include <type_traits>
 
@@ -526,20 +527,9 @@ bool f32_gemm_ok(int type, const uint8_t *w, size_t rb, const float *x, int in_d
     return false;
 }
 
-// Measured for Q6_K: a round of workgroups takes about 6.8 us per super-block on the default tiles and 3.2 on
-// the small ones.
-static bool small_tiles(int out_dim, int m) {
-    const int64_t large = static_cast<int64_t>((out_dim + GeoLarge::kBN - 1) / GeoLarge::kBN) *
-                          ((m + GeoLarge::kBM - 1) / GeoLarge::kBM);
-    return QLIN_F32_GEMM_SMALL && large * 2 < device_info().cu_count;
-}
-float f32_gemm_us_q6k(int out_dim, int in_dim, int m) {
-    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    const bool small = small_tiles(out_dim, m);
-    const int bn = small ? GeoSmall::kBN : GeoLarge::kBN, bm = small ? GeoSmall::kBM : GeoLarge::kBM;
-    const int64_t wgs = static_cast<int64_t>((out_dim + bn - 1) / bn) * ((m + bm - 1) / bm);
-    return 4.0f + static_cast<float>((wgs + cus - 1) / cus) * (small ? 3.2f : 6.8f) * static_cast<float>(in_dim / 256);
-}
+static_assert(GeoLarge::kBM == plan::kSuperLarge.bm && GeoLarge::kBN == plan::kSuperLarge.bn &&
+                  GeoSmall::kBM == plan::kSuperSmall.bm && GeoSmall::kBN == plan::kSuperSmall.bn,
+              "the plan's tiles");
 
 hipError_t f32_gemm(int type, const uint8_t *w, size_t rb, const float *x, float *y, int out_dim, int in_dim, int m,
                     bool add, hipStream_t s) {
@@ -561,7 +551,7 @@ hipError_t f32_gemm(int type, const uint8_t *w, size_t rb, const float *x, float
         else hipLaunchKernelGGL((f32_gemm_kernel<T_Q4_K, G>), grid, dim3(G::kThreads), G::kLdsBytes, s, a);
     };
     // the default tiles, unless they would leave more than half the CUs idle
-    if (small_tiles(out_dim, m)) launch(GeoSmall{});
+    if (QLIN_F32_GEMM_SMALL && plan::super_block_small(out_dim, m, cu_count())) launch(GeoSmall{});
     else launch(GeoLarge{});
     return hipGetLastError();
 }

@@ -505,8 +505,6 @@ static_assert(Large::BM == plan::kGemmLarge.bm && Large::BN == plan::kGemmLarge.
                   Mid::BN == plan::kGemmMid.bn,
               "the plan's tiles");
 
-int cu_count() { return device_info().cu_count > 0 ? device_info().cu_count : 256; }
-
 template <int FMT, bool Q81, int MODE>
 hipError_t by_size(const GemmArgs &a, hipStream_t s) {
     if (plan::gemm(FMT, Q81, a.n, a.k, a.m, MODE == kSwiGLU, cu_count()).large) return launch<FMT, Q81, MODE, Large>(a, s);
@@ -535,10 +533,6 @@ hipError_t run(int type, const GemmArgs &a, bool q81, int mode, hipStream_t s) {
 }
 
 }  // namespace
-
-float gemm_us(int type, bool q81, int n, int k, int m, bool swiglu) {
-    return plan::gemm(type, q81, n, k, m, swiglu, cu_count()).us;
-}
 
 hipError_t gemm_f32(int type, const uint8_t *w0, const uint8_t *w1, size_t rb, const float *x, float *y, int n, int k,
                     int m, int mode, hipStream_t s) {

@@ -79,6 +79,11 @@ hipError_t gemv_generic(int type, const uint8_t *w, size_t rb, const float *x, f
     }
 }
 
+plan::Product rows_product(int type, const uint8_t *w, size_t rb, const float *x, int n, int k, int m) {
+    return plan::product(type, n, k, m, dense_ok(type, w, nullptr, rb, x, n, k), f32_gemm_ok(type, w, rb, x, k),
+                         kF32GemmMinRows, cu_count());
+}
+
 hipError_t gemv(int type, const uint8_t *w, size_t rb, const float *x, float *y, int n, int k, int m,
                 bool add, hipStream_t s) {
     if (n == 0 || m == 0) return hipSuccess;
@@ -86,17 +91,12 @@ hipError_t gemv(int type, const uint8_t *w, size_t rb, const float *x, float *y,
         return mfma_gemv(type, &w, &y, &n, 1, rb, x, k, add, s);
     if (type == T_Q4_K && m == 1 && q4k_stream_ok(&w, 1, rb, x, n, k, false))
         return q4k_stream_gemv(&w, &y, &n, 1, rb, x, k, add, s);
-    if (m > 1 && (type == T_Q4_0 || type == T_Q5_0 || type == T_Q8_0)) {
-        // the prefill GEMM where its tiles fill the chip or x is long enough to be staged once per tile; below
-        // that the waves of a workgroup split K (rows_kernel takes every layout that gets here)
-        const bool dense = dense_ok(type, w, nullptr, rb, x, n, k);
-        if (!dense || gemm_us(type, false, n, k, m, false) < dense_us(type, n, k, m, false))
-            return gemm_f32(type, w, nullptr, rb, x, y, n, k, m, add, s);
+    if (m > 1) switch (rows_product(type, w, rb, x, n, k, m)) {
+        case plan::Product::kGemm: return gemm_f32(type, w, nullptr, rb, x, y, n, k, m, add, s);
+        case plan::Product::kSuperBlockGemm: return f32_gemm(type, w, rb, x, y, n, k, m, add, s);
+        case plan::Product::kDense: return dense_matmul(type, w, nullptr, rb, x, y, n, k, m, add, s);
+        case plan::Product::kPerElement: break;
     }
-    if (m >= kF32GemmMinRows && f32_gemm_ok(type, w, rb, x, k) &&
-        (type != T_Q6_K || !dense_ok(type, w, nullptr, rb, x, n, k) || f32_gemm_us_q6k(n, k, m) <= dense_us(type, n, k, m, false)))
-        return f32_gemm(type, w, rb, x, y, n, k, m, add, s);
-    if (m > 1 && dense_ok(type, w, nullptr, rb, x, n, k)) return dense_matmul(type, w, nullptr, rb, x, y, n, k, m, add, s);
     return gemv_generic(type, w, rb, x, y, n, k, m, add, s);
 }
 

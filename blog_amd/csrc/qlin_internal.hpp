@@ -7,12 +7,15 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "qlin_plan.hpp"
+
 namespace qlin {
 
 struct DeviceInfo {
     int cu_count = 256;
 };
 const DeviceInfo &device_info();
+inline int cu_count() { return device_info().cu_count > 0 ? device_info().cu_count : 256; }
 
 // y[r, o] (=|+=) sum_k W[o, k] x[r, k] for r < m.
 hipError_t gemv(int type, const uint8_t *w, size_t row_bytes, const float *x, float *y, int out_dim,
@@ -103,6 +106,9 @@ bool dense_ok(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, 
 hipError_t dense_matmul(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, float *y,
                         int out_dim, int in_dim, int m, int mode, hipStream_t s, const RouteCombine *combine = nullptr);
 
+// The kernel that gemv() (the GEMV and matmul entry points, plain and adding) takes for m > 1 rows.
+plan::Product rows_product(int type, const uint8_t *w, size_t row_bytes, const float *x, int out_dim, int in_dim, int m);
+
 // MLA over the Q8_1 latent cache (qlin_mla_latent.hip); pos is read from d_pos on the device.
 hipError_t mla_store_latent_q8_1(const float *kv_cache, uint8_t *cache, int kv_lora, int qk_rope, size_t row_bytes,
                                  const int *d_pos, hipStream_t s);
@@ -135,10 +141,7 @@ hipError_t dequant(int type, const uint8_t *src, void *out, int64_t n, bool to_f
 hipError_t quantize_q8_1(const float *x, uint8_t *xq, int in_dim, int m, bool raw_sum, hipStream_t s);
 // The prefill GEMM of the 32-block formats (Q4_0, Q5_0, Q8_0) on the matrix cores (qlin_gemm.hip), products exact:
 // f32 activations (mode 0: y =, 1: y +=, 2: SwiGLU of the gate rows w0 and the up rows w1) or Q8_1 ones, any
-// layout the entry points accept.  gemm_us, dense_us: the estimated microseconds of gemm_f32 (q81: gemm_q8_1) and
-// of dense_matmul (all formats but Q4_K), from which the dispatch chooses.
-float gemm_us(int type, bool q81, int n, int k, int m, bool swiglu);
-float dense_us(int type, int n, int k, int m, bool swiglu);
+// layout the entry points accept.
 hipError_t gemm_f32(int type, const uint8_t *w0, const uint8_t *w1, size_t row_bytes, const float *x, float *y, int n,
                     int k, int m, int mode, hipStream_t s);
 hipError_t gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const uint8_t *xq, float *y, int n, int k, int m,
@@ -154,7 +157,6 @@ hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t row_bytes, const ui
 #define QLIN_F32_GEMM_MIN_ROWS 64
 #endif
 constexpr int kF32GemmMinRows = QLIN_F32_GEMM_MIN_ROWS;
-float f32_gemm_us_q6k(int out_dim, int in_dim, int m);  // its estimated microseconds for Q6_K
 bool f32_gemm_ok(int type, const uint8_t *w, size_t row_bytes, const float *x, int in_dim);
 hipError_t f32_gemm(int type, const uint8_t *w, size_t row_bytes, const float *x, float *y, int out_dim, int in_dim,
                     int m, bool add, hipStream_t s);

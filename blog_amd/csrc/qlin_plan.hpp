@@ -96,11 +96,12 @@ inline int64_t tiles(int n, int bn, int m, int bm) {
 
 // The row products of qlin_dense.hip (rows_kernel): nt row tiles (of a SwiGLU: nt / 2 outputs') by tt token tiles
 // of 16 per workgroup, one workgroup on a CU at a time, whose 8 waves take units of 128 values of K in turn.
-// us is `base` plus, per round of workgroups, round + unit x (units of a wave): least squares of the logarithm over
-// the tiles of 36 shapes of each format (n 512 .. 32768, k 512 .. 16384, m 2 .. 700), 9-10% off in the mean; the
-// kernel it picks is at most 0.4% slower in the mean than the fastest, and 13% at one shape.  Larger tiles split x and read the
-// weights for more products, smaller ones fill the chip.  Q6_K has no 2 x 4 tiles (they spill: 8.0 us a unit, as
-// much per product as 2 x 3's 5.7).
+// us is base plus, per round of workgroups, round + unit x (the units of K / 8: a tenth of it rounded up to whole
+// turns of the waves), by least squares of the logarithm over the tiles of 61 shapes of each format (36 of n 512 ..
+// 32768, k 512 .. 16384, m 2 .. 700; full rounds of k 1024 .. 16384; 13 of k 32 .. 512, not of Q6_K): 5-7% off in
+// the mean; the kernel and tiles it picks are 0.1-0.2% slower in the mean than the fastest, 10% at worst.  Larger
+// tiles split x and read the weights for more products, smaller ones fill the chip.  Q6_K has no 2 x 4 tiles (they
+// spill: 8.2 us a unit, as much per product as 2 x 3's 6.0), the others no 1 x 2 (the cheapest for 6 of 10000 shapes).
 struct Rows {
     int nt = 0, tt = 0;
     float us = 0.0f;
@@ -109,16 +110,17 @@ inline Rows rows(int type, int n, int k, int m, bool swiglu, int cus) {
     static constexpr int nt[6] = {1, 2, 1, 2, 2, 2}, tt[6] = {1, 1, 2, 2, 3, 4};
     static constexpr struct {
         float base, round[6], unit[6];
-    } costs[4] = {{0.75f, {0.95f, 1.55f, 1.4f, 2.4f, 3.1f, 3.3f}, {1.45f, 1.98f, 2.42f, 3.1f, 4.1f, 5.2f}},
-                  {0.8f, {0.9f, 1.6f, 1.55f, 2.3f, 2.9f, 3.6f}, {1.63f, 2.31f, 2.58f, 3.5f, 4.6f, 5.6f}},
-                  {0.8f, {1.2f, 1.5f, 1.35f, 2.2f, 2.7f, 3.55f}, {1.55f, 2.41f, 2.64f, 3.5f, 4.5f, 5.6f}},
-                  {1.45f, {0.95f, 1.15f, 1.25f, 1.4f, 2.45f, 0.0f}, {1.83f, 3.2f, 2.86f, 4.55f, 5.7f, 0.0f}}};
+    } costs[4] = {{1.15f, {1.3f, 1.85f, 0.0f, 2.75f, 3.7f, 4.55f}, {1.51f, 2.13f, 0.0f, 3.36f, 4.38f, 5.4f}},
+                  {1.0f, {1.4f, 2.0f, 0.0f, 2.95f, 3.95f, 5.0f}, {1.65f, 2.46f, 0.0f, 3.68f, 4.76f, 5.81f}},
+                  {1.1f, {1.3f, 1.7f, 0.0f, 2.6f, 3.55f, 4.6f}, {1.68f, 2.65f, 0.0f, 3.95f, 5.0f, 6.24f}},
+                  {1.3f, {1.35f, 1.85f, 1.9f, 2.45f, 3.55f, 0.0f}, {1.93f, 3.34f, 2.96f, 4.69f, 5.98f, 0.0f}}};
     const int f = rows_format(type);
     Rows best;
     if (f < 0) return best;
-    const float units = static_cast<float>((k / 32 + 31) / 32);
-    for (int i = 0; i < (f == 3 ? 5 : 6); ++i) {
-        if (swiglu && nt[i] == 1) continue;
+    const int all = (k / 32 + 3) / 4;
+    const float units = 0.1f * static_cast<float>((all + 7) / 8) + 0.1125f * static_cast<float>(all);
+    for (int i = 0; i < 6; ++i) {
+        if (i == (f == 3 ? 5 : 2) || (swiglu && nt[i] == 1)) continue;
         const int64_t wgs = tiles(n, 16 * nt[i] / (swiglu ? 2 : 1), m, 16 * tt[i]);
         const float us = costs[f].base + static_cast<float>((wgs + cus - 1) / cus) * (costs[f].round[i] + units * costs[f].unit[i]);
         if (!best.nt || us < best.us) {
@@ -131,7 +133,7 @@ inline Rows rows(int type, int n, int k, int m, bool swiglu, int cus) {
 }
 
 // The prefill GEMM (qlin_gemm.hip): its tiles (bm tokens x bn rows) and the microseconds of a launch, fill + K steps
-// of 64 x the cost of one, fitted as above (4-9% off in the mean): with the large tiles a step per round of
+// of 64 x the cost of one, fitted as above (5-9% off in the mean): with the large tiles a step per round of
 // workgroups; with the middle ones a step of one workgroup on a CU, or of two at a time, which LDS and registers
 // have room for.
 struct Tile {
@@ -145,7 +147,7 @@ struct Gemm {
 inline Gemm gemm(int type, bool q81, int n, int k, int m, bool swiglu, int cus) {
     static constexpr struct {
         float fill, step, mid_fill, mid_two, mid_one;
-    } costs[2][3] = {{{7.3f, 2.5f, 2.8f, 2.08f, 1.41f}, {8.3f, 2.57f, 2.8f, 2.22f, 1.56f}, {7.8f, 2.48f, 2.4f, 1.98f, 1.52f}},
+    } costs[2][3] = {{{6.3f, 2.56f, 3.35f, 2.15f, 1.4f}, {6.8f, 2.65f, 3.35f, 2.28f, 1.55f}, {7.0f, 2.54f, 3.3f, 2.27f, 1.51f}},
                      {{7.5f, 1.67f, 1.85f, 1.3f, 0.86f}, {7.6f, 1.71f, 2.6f, 1.41f, 0.99f}, {7.1f, 1.69f, 1.75f, 1.17f, 1.07f}}};
     const int f = rows_format(type);
     if (f < 0 || f > 2) return Gemm{};
@@ -200,6 +202,40 @@ inline Q81 q8_1_route(int type, int n, int k, int m, bool qblk_ok, bool gemm_ok,
 inline bool rows_layout_ok(int type, uintptr_t w0, uintptr_t w1, size_t row_bytes, uintptr_t x, int n, int k) {
     return rows_format(type) >= 0 && k % (type == 14 ? 256 : 32) == 0 && (n <= 1 || row_bytes % 2 == 0) && w0 % 2 == 0 &&
            w1 % 2 == 0 && x % 4 == 0;
+}
+
+// The prefill GEMM of the super-block formats (qlin_f32_gemm.hip): the default tiles, unless they would leave more
+// than half the CUs idle, and the microseconds of a Q6_K launch (a round of workgroups takes about 6.8 us per
+// super-block on the default tiles and 3.2 on the small ones).
+constexpr Tile kSuperLarge{64, 256}, kSuperSmall{32, 128};
+inline bool super_block_small(int n, int m, int cus) { return tiles(n, kSuperLarge.bn, m, kSuperLarge.bm) * 2 < cus; }
+inline float super_block_us(int n, int k, int m, int cus) {
+    const bool s = super_block_small(n, m, cus);
+    const Tile t = s ? kSuperSmall : kSuperLarge;
+    return 4.0f + static_cast<float>((tiles(n, t.bn, m, t.bm) + cus - 1) / cus) * (s ? 3.2f : 6.8f) * static_cast<float>(k / 256);
+}
+
+// The kernel of a product with m > 1 rows of f32 activations, as dense_matmul (kDense: rows_kernel, Q4_K's own) and the
+// GEMMs take the layout: the GEMM of the 32-block formats where its tiles fill the chip or x is long enough to be
+// staged once per tile (below that the waves of a workgroup split K), that of the super-block formats from min_rows
+// rows on (Q6_K: where it is the cheaper one; Q4_K's dense_matmul holds less of x).
+enum class Product { kPerElement, kDense, kGemm, kSuperBlockGemm };
+inline Product product(int type, int n, int k, int m, bool dense_ok, bool super_block_ok, int min_rows, int cus) {
+    const int f = rows_format(type);
+    if (f >= 0 && f < 3)
+        return !dense_ok || gemm(type, false, n, k, m, false, cus).us < rows(type, n, k, m, false, cus).us ? Product::kGemm
+                                                                                                       : Product::kDense;
+    if (m >= min_rows && super_block_ok &&
+        (f < 0 || !dense_ok || super_block_us(n, k, m, cus) <= rows(type, n, k, m, false, cus).us))
+        return Product::kSuperBlockGemm;
+    return dense_ok ? Product::kDense : Product::kPerElement;
+}
+// The same of a SwiGLU over m > 1 rows (no GEMM of the super-block formats has that mode).
+inline Product swiglu_product(int type, int ffn, int k, int m, bool dense_ok, int cus) {
+    const int f = rows_format(type);
+    if (f >= 0 && f < 3 && (!dense_ok || gemm(type, false, ffn, k, m, true, cus).us < rows(type, ffn, k, m, true, cus).us))
+        return Product::kGemm;
+    return dense_ok ? Product::kDense : Product::kPerElement;
 }
 
 }  // namespace plan

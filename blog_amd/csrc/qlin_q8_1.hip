@@ -56,9 +56,8 @@ hipError_t matmul_q8_1(int type, const uint8_t *w, size_t rb, const uint8_t *xq,
     if (waves == 0) return hipSuccess;
     if (type == T_Q4_K && q4k_gemm_ok(w, rb, xq, in_dim)) return q4k_gemm_q8_1(w, rb, xq, y, out_dim, in_dim, m, s);
     if (type == T_Q4_0 || type == T_Q5_0 || type == T_Q8_0) {
-        const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
         const plan::Q81 route = plan::q8_1_route(type, out_dim, in_dim, m, qblk_gemm_ok(type, w, rb, xq, in_dim),
-                                                 (reinterpret_cast<uintptr_t>(xq) & 3u) == 0, cus);
+                                                 (reinterpret_cast<uintptr_t>(xq) & 3u) == 0, cu_count());
         if (route == plan::Q81::kGemm) return gemm_q8_1(type, w, rb, xq, y, out_dim, in_dim, m, s);
     }
     if (qblk_gemm_ok(type, w, rb, xq, in_dim)) return qblk_gemm_q8_1(type, w, rb, xq, y, out_dim, in_dim, m, s);

@@ -618,7 +618,6 @@ bool qblk_gemm_ok(int type, const uint8_t *w, size_t rb, const uint8_t *xq, int 
 static_assert(GeoLarge::kBM == plan::kQblkLarge.bm && GeoLarge::kBN == plan::kQblkLarge.bn &&
                   GeoSmall::kBM == plan::kQblkSmall.bm && GeoSmall::kBN == plan::kQblkSmall.bn,
               "the plan's tiles");
-static int cu_count() { return device_info().cu_count > 0 ? device_info().cu_count : 256; }
 static bool small_tiles(int out_dim, int m) { return QLIN_QBLK_SMALL && plan::qblk_small(out_dim, m, cu_count()); }
 
 hipError_t qblk_gemm_q8_1(int type, const uint8_t *w, size_t rb, const uint8_t *xq, float *y, int out_dim,

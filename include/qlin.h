@@ -305,9 +305,9 @@ int qlin_moe_routed_decode_grouped_logits(int gate_up_type, const uint8_t *gate_
  * logits.  out [tokens, hidden_size] gets (out + the routed sum) + the shared experts' down projection
  * of SiLU(shared gate x) * (shared up x), each token's result exactly that of
  * qlin_moe_routed_decode_grouped_logits followed by qlin_launch_quant_swiglu_rows and
- * qlin_launch_quant_matmul_add on the shared weights, which is what the call runs when the shared
- * down projection cannot take the m > 1 matrix-core kernel; when it can (tokens > 1), that launch
- * also adds the routed sum, so the separate combine launch is not needed.  Shared weights:
+ * qlin_launch_quant_matmul_add on the shared weights, which is what the call runs when the last of
+ * them takes the decode GEMV or a prefill GEMM; when it takes the kernel for a few rows (tokens > 1), that
+ * launch also adds the routed sum, so the separate combine launch is not needed.  Shared weights:
  * gate and up [shared_ffn, in_dim] of shared_type with rows of shared_gate_up_row_bytes, down
  * [hidden_size, shared_ffn] with rows of shared_down_row_bytes; shared_ffn = 0 runs the routed part
  * alone.  workspace: at least qlin_moe_ffn_workspace_bytes(...) bytes, 256-byte aligned (the routed

@@ -488,13 +488,17 @@ def test_f32_gemm_prefill_shape_every_row(qtype, N, K, M):
     assert row_err.max() <= 1e-5, (int(row_err.argmax()), float(row_err.max()))
 
 
-@pytest.mark.parametrize("qtype", [Q4_K, Q6_K])
-def test_f32_gemm_token_scales(qtype):
-    """The prefill GEMM scales each token's 256 values of a super-block by a power of two into the
+# (type, N, K, m) that take the prefill GEMM of the super-block formats (tests/test_plan.py)
+F32_GEMM_SCALES = [(Q4_K, 300, 1024, 70), (Q6_K, 8192, 1024, 70)]
+F32_GEMM_ADD = [(Q4_K, 520, 2048, 64), (Q4_K, 520, 2048, 96), (Q6_K, 8192, 2048, 96)]
+
+
+@pytest.mark.parametrize("qtype,N,K,M", F32_GEMM_SCALES)
+def test_f32_gemm_token_scales(qtype, N, K, M):
+    """The prefill GEMM of the super-block formats scales each token's 256 values of a super-block by a power of two into the
     fp16 range: tokens whose values span 1e-30 .. 1e30, an all-zero token, a token with one huge
     value among tiny ones and a super-block of zeros inside a token, each within 1e-5 of the f64
     oracle relative to that token's own largest output (a shared scale would lose the small ones)."""
-    N, K, M = 300, 1024, 70
     w, rb, vals = qgen.random_matrix(qtype, N, K, seed=95)
     rng = np.random.default_rng(96)
     x = rng.standard_normal((M, K)).astype(np.float32)
@@ -519,10 +523,9 @@ def test_f32_gemm_token_scales(qtype):
         assert err <= COND, (i, float(err))
 
 
-@pytest.mark.parametrize("qtype,m", [(Q4_K, 64), (Q4_K, 96), (Q6_K, 96)])
-def test_f32_gemm_add(qtype, m):
+@pytest.mark.parametrize("qtype,N,K,m", F32_GEMM_ADD)
+def test_f32_gemm_add(qtype, N, K, m):
     """y += W x over m >= 64 tokens (launch_quant_matmul's add form) on the prefill GEMM."""
-    N, K = 520, 2048
     w, rb, _ = qgen.random_matrix(qtype, N, K, seed=97 + m)
     x = qgen.random_x(m, K, seed=98 + m)
     y0 = np.random.default_rng(99).standard_normal((m, N)).astype(np.float32)
@@ -533,18 +536,26 @@ def test_f32_gemm_add(qtype, m):
     assert normwise_rel_err(host(yd), ref) <= FP32
 
 
-BLOCK_ROWS = [  # (type, N, K, m): few rows and short K (a unit of blocks cut short), every tile kind, odd block counts
-    (Q8_0, 100, 96, 2), (Q5_0, 33, 1056, 17), (Q4_0, 520, 160, 40), (Q8_0, 1718, 1280, 25), (Q4_0, 4000, 544, 70),
-    (Q6_K, 70, 256, 5), (Q6_K, 300, 1280, 33), (Q6_K, 1030, 768, 130),
-    (Q8_0, 8300, 224, 130),      # the GEMM's 64 x 128 tiles, 7 blocks
-    (Q5_0, 14400, 2080, 260),    # its 128 x 256 tiles, 65 blocks
-    (Q4_0, 14400, 2048, 300),
-    (Q8_0, 8300, 224, 270),      # two workgroups on a CU
-    (Q8_0, 890, 160, 370), (Q5_0, 890, 1056, 370), (Q4_0, 890, 160, 370), (Q6_K, 900, 256, 380)]  # 2 x 3 tiles
+# (type, N, K, m, the kernel it takes at 256 CUs, that of its SwiGLU): row tiles x token tiles of rows_kernel, the
+# middle and the large tiles of the prefill GEMM (tests/test_plan.py checks the names).  Few rows and short K (a
+# unit of blocks cut short), every tile kind of every format, odd block counts, remainders of tiles.
+BLOCK_ROWS = [
+    (Q8_0, 100, 96, 2, "1x1", "2x1"), (Q5_0, 33, 1056, 17, "1x1", "2x1"), (Q4_0, 520, 160, 40, "1x1", "2x1"),
+    (Q8_0, 1718, 1280, 25, "1x1", "2x1"), (Q4_0, 4000, 544, 70, "2x3", "2x3"), (Q6_K, 70, 256, 5, "1x1", "2x1"),
+    (Q6_K, 300, 1280, 33, "1x1", "2x1"), (Q6_K, 1030, 768, 130, "2x2", "2x3"), (Q6_K, 2744, 512, 23, "1x2", "2x2"),
+    (Q6_K, 5000, 512, 12, "2x1", "2x1"), (Q8_0, 5000, 512, 12, "2x1", "2x1"), (Q5_0, 5000, 512, 12, "2x1", "2x1"),
+    (Q4_0, 5000, 512, 12, "2x1", "2x1"), (Q8_0, 4000, 512, 60, "2x2", "2x4"), (Q5_0, 4000, 512, 60, "2x2", "2x4"),
+    (Q4_0, 4000, 512, 60, "2x2", "2x4"), (Q8_0, 4100, 1056, 60, "2x4", "2x2"), (Q5_0, 4100, 1056, 60, "2x4", "2x2"),
+    (Q4_0, 4100, 1056, 60, "2x4", "2x2"), (Q8_0, 890, 160, 370, "2x3", "mid"), (Q8_0, 890, 1056, 370, "2x3", "2x3"),
+    (Q5_0, 890, 1056, 370, "2x3", "2x3"), (Q4_0, 890, 160, 370, "2x3", "mid"), (Q6_K, 900, 256, 380, "2x3", "2x3"),
+    (Q8_0, 8300, 224, 130, "mid", "mid"), (Q5_0, 8300, 224, 130, "mid", "mid"), (Q4_0, 8300, 224, 130, "mid", "mid"),
+    (Q8_0, 8300, 224, 270, "mid", "large"),  # (two workgroups on a CU)
+    (Q5_0, 14400, 2080, 260, "large", "large"), (Q4_0, 14400, 2048, 300, "large", "large"),
+    (Q8_0, 14400, 1056, 300, "large", "large")]
 
 
 @pytest.mark.parametrize("mode", ["store", "add", "swiglu"])
-@pytest.mark.parametrize("qtype,N,K,m", BLOCK_ROWS)
+@pytest.mark.parametrize("qtype,N,K,m", [c[:4] for c in BLOCK_ROWS])
 def test_rows_of_f32(qtype, N, K, m, mode):
     """Several rows of f32 activations (quant_matmul, its add form, the SwiGLU rows): against the f64 oracle, each output within 2e-5 of its own sum |w||x| (the bound of the other
     f32 paths) and normwise 1e-5."""
@@ -1118,6 +1129,8 @@ def test_moe_grouped_unaligned_output():
     (Q4_K, 8, 20, 2, 256, 512, 512, Q4_K),      # over 16 tokens: the shared SwiGLU as its own launch
     (Q4_K, 8, 6, 2, 256, 512, 4352, Q4_K),      # 272 shared tiles on 136 workgroups, two each
     (Q4_K, 8, 6, 2, 256, 512, 8448, Q4_K),      # 528 shared tiles, more than two per workgroup: its own launch
+    (Q4_K, 8, 70, 2, 256, 512, 512, Q4_K),      # 64 tokens and more: the shared down is a prefill GEMM
+    (Q4_K, 8, 300, 2, 256, 2304, 96, Q8_0),     # so many that the 32-block formats' is one, too
 ])
 def test_moe_ffn_matches_three_calls(gu, E, tokens, k, ffn, hid, sffn, stype):
     """The MoE FFN call (routed from the logits, then the shared experts) gives, bit for bit, what the
