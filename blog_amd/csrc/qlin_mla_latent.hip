@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kCThreads) void context_kernel(const ContextArgs a)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const bool in = t0 + 4 * g + i <= pos;
-            const float e = in ? __expf(cur.s[i] - mx) : 0.0f;
+            const float e = in ? expf(cur.s[i] - mx) : 0.0f;
             den += e;
             const uint32_t q = cur.q[i] & qmask;
             const float d = f16_bits_to_f32(cur.ds[i] & 0xffffu);

@@ -214,6 +214,31 @@ def test_scores_and_context(n_heads, T, pos):
 
 
 @pytest.mark.gpu
+def test_context_exponentials():
+    """context's softmax takes expf, whose error does not grow with the distance from the maximum: with a zero
+    latent row at the maximum, what is left lies 20 to 65 below it, and each output of a head (one position's
+    share of it; the others vanish) is right to a few roundings (expf, its product, the sums and the
+    division: 5 x 2^-24 = 3e-7; the fast exponential is off by up to |s - max| 2^-24 = 4e-6)."""
+    from gpu_util import banner, bind_stream, dev, empty_f32, host
+    n_heads, T, pos = 32, 16, 8
+    kv, cache, crb = make_cache(T, KL, QR, 140)
+    cache[0] = 0
+    rng = np.random.default_rng(141)
+    s = np.full((n_heads, T), -400.0, np.float32)
+    s[:, 0] = 0.0                                                            # (differences exact)
+    s[:, 1] = -rng.uniform(20, 65, n_heads)
+    banner("mla context exponentials")
+    bind_stream()
+    lat_d, dl_d = empty_f32(n_heads, KL), empty_f32(n_heads, KL // 32)
+    qlin.call("qlin_launch_mla_absorb_context_device_pos", dev(s), dev(cache), crb, dl_d, lat_d, n_heads, KL, _pos(pos), T)
+    lat, dl = orc.mla_absorb_context(s, cache, crb, n_heads, KL, pos, T)
+    for got, ref in ((host(lat_d), lat), (host(dl_d), dl)):
+        ref = ref.astype(np.float64)
+        err = np.max(np.abs(got - ref), axis=1) / np.max(np.abs(ref), axis=1)
+        assert err.max() <= 6e-7, float(err.max())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,pos", [(256, 0), (256, 255), (1024, 700)])
 def test_attend_fused(T, pos):
     from gpu_util import banner, bind_stream, dev, empty_f32, host
