@@ -238,5 +238,10 @@ inline Product swiglu_product(int type, int ffn, int k, int m, bool dense_ok, in
     return dense_ok ? Product::kDense : Product::kPerElement;
 }
 
+// Workgroups of the Q8_1 quantizer (8 lanes per block, 32 blocks at a time): at most kQuantizeGroups, which then take
+// further blocks in turn, since a launch's threads have to stay below 2^32 (2^29 blocks, 64 GiB of x).
+constexpr int64_t kQuantizeGroups = int64_t{1} << 16;
+inline int64_t quantize_groups(int64_t blocks) { return std::min(kQuantizeGroups, (blocks + 31) / 32); }
+
 }  // namespace plan
 }  // namespace qlin

@@ -79,6 +79,12 @@ int main() {
         CHECK(!c.ok);
         CHECK(!stream(q4k, true, 16, 256, 64, 6, 256, kMaxLds, kMaxLds).ok);  // unreadable kernels
     }
+    // the quantizer's launch: a group per 32 blocks, its threads below 2^32 however many blocks there are
+    for (int64_t blocks : {int64_t{1}, int64_t{33}, int64_t{1} << 20, int64_t{1} << 29, int64_t{1} << 31, int64_t{1} << 40}) {
+        const int64_t g = quantize_groups(blocks);
+        CHECK(g >= 1 && g <= (blocks + 31) / 32 && g * 256 < (int64_t{1} << 32));
+        CHECK(g == (blocks + 31) / 32 || g == kQuantizeGroups);
+    }
     // Q8_1 products in layouts that the 64-token GEMM does not take: few outputs stay with the block dots,
     // however long their rows; enough of them take the other GEMM.  (Q4_0 2, Q5_0 6, Q8_0 8)
     for (int type : {2, 6, 8}) {

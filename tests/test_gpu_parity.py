@@ -369,6 +369,16 @@ def test_quantize_q8_1_bit_exact(raw):
     assert np.array_equal(host(xq), orc.quantize_q8_1(x, in_dim, raw))
 
 
+def test_quantize_q8_1_more_blocks_than_a_launch_has_lanes_for():
+    """Over 2^21 blocks, past which the quantizer's workgroups take several each."""
+    in_dim, m = 7, (1 << 21) + 77
+    x = qgen.random_x(m, in_dim, seed=17)
+    banner(f"quantize q8_1 {m} blocks")
+    xq = torch.zeros(m * 36, dtype=torch.uint8, device="cuda")
+    qlin.quantize_q8_1(dev(x), xq, in_dim, m)
+    assert np.array_equal(host(xq), orc.quantize_q8_1(x.reshape(-1), in_dim))
+
+
 @pytest.mark.parametrize("qtype,out_dim,in_dim,m", [(Q4_K, 96, 1024, 7), (Q6_K, 40, 512, 3), (Q8_0, 50, 256, 4),
                                                     (Q5_0, 33, 128, 2), (Q4_0, 17, 64, 3), (Q4_K, 512, 4096, 64),
                                                     (Q4_K, 300, 768, 70), (Q4_K, 257, 256, 1),
