@@ -472,10 +472,13 @@ int qlin_launch_attend(const float *q, const float *key_cache, const float *valu
     if (!qlin::al16(q) || !qlin::al16(key_cache) || !qlin::al16(value_cache) || !qlin::al16(attn) ||
         !qlin::al4(start_pos_dev))
         return QLIN_ERR_ALIGN;
-    // Whole groups of 16 rows, and enough (row, head) pairs that attend_kernel's workgroups would wait for one
-    // another: the position is not known here, and from 448 pairs on attend_rows_kernel is the faster one from
-    // the cache's start to its end (32 rows of 14 heads at 0: 6.0 -> 5.2 us, at 1500: 39.2 -> 29.8; 16 rows of
-    // 32 heads of 128 at 3000: 146 -> 111), while 16 rows of 14 heads at 1500 take 26.9 us there and 29.6 here.
+    // Whole groups of 16 rows, and so many (row, head) pairs that attend_kernel's workgroups, one each, wait for one
+    // another (up to 256 every CU has its own), while attend_rows_kernel takes the same time until its tiles fill
+    // the chip.  The position is not known here.  Measured over 4 .. 64 heads of 64 and 128, 16 .. 128 rows, positions 0 ..
+    // 7900 (attend_kernel, attend_rows_kernel, us): 256 pairs (32 rows of 8 heads of 64) 8.0, 9.8 at 200 and 59, 70 at
+    // 4000; 448 (32 rows of 14 heads) 6.2, 5.6 at 0, 10.0, 9.8 at 200 and 90, 71 at 4000; 448 of 128 (16 rows of 28 heads)
+    // 7.4, 7.2 and 14.5, 15.6 and 181, 147; 512 (128 rows of 4 heads of 128, the worst) 9.9, 12.1 at 0, 21.9, 18.8 at 200;
+    // 2048 (64 rows of 32 heads of 128) 15.9, 8.9 and 52, 18 and 747, 139.
     if (rows >= 16 && static_cast<int64_t>(rows) * n_heads >= 448 && (head_dim == 64 || head_dim == 128)) {
         const dim3 grid((rows + 15) / 16, n_heads), block(64 * qlin::kRowWaves);
         if (head_dim == 64)

@@ -433,11 +433,20 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
                 }
                 return;
             }
+            // (the unit's own sum, then added: a shorter chain of roundings)
             const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            f32x4 sum[NT];
 #pragma unroll
             for (int j = 0; j < kUnit; ++j) {
                 u32x4 hi, mid, lo;
                 split3(x[2 * j], x[2 * j + 1], hi, mid, lo);
+                auto scaled = [&](const f32x4 (&D)[NT], int scale) {
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            sum[t][r] = scale ? fmaf(dw[t][scale], D[t][r], sum[t][r]) : dw[t][0] * D[t][r];
+                };
                 if constexpr (Q6) {
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
@@ -448,10 +457,7 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
                         for (int t = 0; t < NT; ++t) D[t] = mfma16(mid[2 * s], mid[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], D[t]);
 #pragma unroll
                         for (int t = 0; t < NT; ++t) D[t] = mfma16(hi[2 * s], hi[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], D[t]);
-#pragma unroll
-                        for (int t = 0; t < NT; ++t)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][2 * j + s], D[t][r], acc[i][t][r]);
+                        scaled(D, 2 * j + s);
                     }
                 } else {
                     f32x4 D[NT];
@@ -461,14 +467,14 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
                     for (int t = 0; t < NT; ++t) D[t] = mfma(mid, B[t][j], D[t]);
 #pragma unroll
                     for (int t = 0; t < NT; ++t) D[t] = mfma(hi, B[t][j], D[t]);
-#pragma unroll
-                    for (int t = 0; t < NT; ++t)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(dw[t][j], D[t][r], acc[i][t][r]);
+                    scaled(D, j);
                 }
             }
 #pragma unroll
-            for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(acc[i][t]));  // (not sunk below the next tile)
+            for (int t = 0; t < NT; ++t) {
+                acc[i][t] += sum[t];
+                asm volatile("" : "+v"(acc[i][t]));  // (not sunk below the next tile)
+            }
         };
         tile(0);
         if constexpr (TT > 1) tile(1);
