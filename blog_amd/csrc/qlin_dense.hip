@@ -184,9 +184,9 @@ __global__ __launch_bounds__(kDThreads) void q4k_dense_kernel(const DenseArgs a)
 // What bounds it: a tile's chain (x turned in LDS, 176 instructions to split its 32 values a lane, 12-24 MFMAs and
 // their scaling) with two or three waves on a SIMD.  Against f32 matrix cores (v_mfma_f32_16x16x4_f32) on decoded
 // values: Q6_K [3584, 18944] at 12 rows 78 -> 33 us, Q5_0 [4096, 4096] at 6 rows 18.4 -> 9.2 us, Q8_0 [4096, 4096]
-// at 100 rows 107 -> 32 us; 2-norm error against f64 over N(0, 1) x of 2048 values 2.9e-7 -> 0.9e-7 (1.0e-7 as an
-// fp16 pair under a scale per token, at the same times).  149 registers (1 x 1) to 256 (2 x 4: 0 to 6 of them
-// spilled, Q6_K's 2 x 3 up to 2; the measured costs in qlin_plan.hpp include them).
+// at 100 rows 107 -> 32 us; 2-norm error against f64 over N(0, 1) x 2.1e-7 .. 8.6e-7 -> 0.8e-7 .. 1.2e-7 (0.9e-7 .. 1.6e-7
+// as an fp16 pair under a scale per token, at the same times).  149 registers (1 x 1) to 256 (2 x 4: 0 to 6 of them
+// spilled, Q6_K's 2 x 3 up to 4; the measured costs in qlin_plan.hpp include them).
 
 constexpr int kUnit = 4;  // 32-blocks of a unit
 

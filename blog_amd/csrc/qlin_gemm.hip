@@ -1,5 +1,5 @@
 // qlin_gemm.hip -- the prefill GEMM of the 32-block formats: Q8_0, Q5_0 and Q4_0 weights times many rows of
-// activations, f32 or Q8_1, on the fp16 matrix cores of gfx950.
+// activations, f32 or Q8_1, on the matrix cores of gfx950.
 //
 //   y[r, o] (=|+=) sum_k w(o, k) x[r, k]                          (kernel.cu:1254-1279, quant_matmul_kernel)
 //   y[r, o]  =     sum over 32-blocks of the Q8_1 block dots      (kernel.cu:2305-2402, quant_matmul_q8_1)

@@ -5,9 +5,9 @@
 // kernel.cu:1192-1244).  The summation order is ours (results agree within fp32 rounding).
 //
 // m == 1 goes to the matrix-core decode kernels (qlin_mfma_gemv.hip) or the streaming Q4_K kernel
-// (qlin_q4k_stream.hip), Q4_K with m > 1 to the f32 matrix-core kernel (qlin_dense.hip); everything
-// else takes the generic per-element kernel below, which decodes each weight with the reference's
-// per-element formula.
+// (qlin_q4k_stream.hip), m > 1 to the row products (qlin_dense.hip) or a prefill GEMM (qlin_gemm.hip,
+// qlin_f32_gemm.hip) by plan::product; layouts that none of them reads take the generic per-element kernel
+// below, which decodes each weight with the reference's per-element formula.
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
 
