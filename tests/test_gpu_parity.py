@@ -720,6 +720,36 @@ def test_rows_of_f32_over_the_whole_range(qtype, N, m):
     assert (got[6][w0 != 0] == -np.sign(w0[w0 != 0]) * np.inf).all()
 
 
+@pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 100, 256, 9), (Q5_0, 100, 256, 9), (Q4_0, 100, 256, 9),
+                                         (Q6_K, 100, 512, 9), (Q8_0, 8300, 224, 130), (Q4_0, 14400, 1056, 300)])
+def test_rows_of_f32_infinite_block_scale(qtype, N, K, m):
+    """A block scale of infinity makes each of its weights infinite, or NaN where the integer is 0: the sum is
+    infinite where all of them push one way and NaN otherwise, in its own row alone."""
+    w, rb, vals = qgen.random_matrix(qtype, N, K, seed=495)
+    b = w.reshape(N, rb)
+    at = {Q8_0: 0, Q5_0: 0, Q4_0: 0, Q6_K: 208}[qtype]
+    for row in (1, N - 2):                         # the largest integer all over block 0
+        b[row, :qgen.BLOCK[qtype][1]] = 0x7f if qtype == Q8_0 else 0xff
+        if qtype == Q6_K:
+            b[row, 192:208] = 1
+    for row in (1, 5, N - 2):
+        b[row, at:at + 2] = (0x00, 0x7c)
+    x = qgen.random_x(m, K, seed=496)
+    x[::2] = np.abs(x[::2]) + np.float32(0.1)
+    banner(f"rows infinite scale type={qtype} {m}x{K}x{N}")
+    yd = empty_f32(m, N)
+    qlin.quant_matmul(qtype, dev(w), rb, dev(x), yd, N, K, m)
+    got = host(yd)
+    for row in (1, N - 2):
+        assert (got[::2, row] == np.inf).all() and np.isnan(got[1::2, row]).all()
+    assert np.isnan(got[:, 5]).all()               # (random integers of both signs)
+    rest = np.setdiff1d(np.arange(N), (1, 5, N - 2))
+    assert np.isfinite(got[:, rest]).all()
+    toks = np.unique(np.r_[0, 1, m - 1])
+    ref = x[toks].astype(np.float64) @ vals[rest].astype(np.float64).T
+    assert normwise_rel_err(got[toks][:, rest], ref) <= FP32
+
+
 @pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 14400, 1088, 257), (Q5_0, 14400, 1024, 130), (Q4_0, 70, 96, 5),
                                          (Q8_0, 300, 1056, 66)])
 def test_matmul_q8_1_shared_gemm(qtype, N, K, m):
