@@ -184,9 +184,9 @@ __global__ __launch_bounds__(kDThreads) void q4k_dense_kernel(const DenseArgs a)
 // What bounds it: a tile's chain (x turned in LDS, 176 instructions to split its 32 values a lane, 12-24 MFMAs and
 // their scaling) with two or three waves on a SIMD.  Against f32 matrix cores (v_mfma_f32_16x16x4_f32) on decoded
 // values: Q6_K [3584, 18944] at 12 rows 78 -> 33 us, Q5_0 [4096, 4096] at 6 rows 18.4 -> 9.2 us, Q8_0 [4096, 4096]
-// at 100 rows 107 -> 32 us; 2-norm error against f64 over N(0, 1) x 2.1e-7 .. 8.6e-7 -> 0.8e-7 .. 1.2e-7 (0.9e-7 .. 1.6e-7
+// at 100 rows 107 -> 32 us; 2-norm error against f64 over N(0, 1) x 2.1e-7 .. 8.6e-7 -> 0.7e-7 .. 1.2e-7 (0.9e-7 .. 1.6e-7
 // as an fp16 pair under a scale per token, at the same times).  149 registers (1 x 1) to 256 (2 x 4: 0 to 6 of them
-// spilled, Q6_K's 2 x 3 up to 4; the measured costs in qlin_plan.hpp include them).
+// spilled, Q6_K's 2 x 3 up to 6; the measured costs in qlin_plan.hpp include them).
 
 constexpr int kUnit = 4;  // 32-blocks of a unit
 
@@ -452,21 +452,25 @@ __global__ __launch_bounds__(kDThreads) void rows_kernel(const DenseArgs a) {
                     for (int s = 0; s < 2; ++s) {
                         f32x4 D[NT];
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) D[t] = mfma16(lo[2 * s], lo[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], zero);
+                        for (int t = 0; t < NT; ++t) D[t] = mfma16(hi[2 * s], hi[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], zero);
 #pragma unroll
                         for (int t = 0; t < NT; ++t) D[t] = mfma16(mid[2 * s], mid[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], D[t]);
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) D[t] = mfma16(hi[2 * s], hi[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], D[t]);
+                        for (int t = 0; t < NT; ++t) D[t] = mfma16(lo[2 * s], lo[2 * s + 1], B[t][j][2 * s], B[t][j][2 * s + 1], D[t]);
                         scaled(D, 2 * j + s);
                     }
                 } else {
-                    f32x4 D[NT];
+                    // the small parts' sum apart from hi's: 0.7e-7 .. 0.9e-7 from f64 instead of 1.0e-7 .. 1.1e-7, for 1-3%
+                    // of the time (Q6_K's sums are half as long: 1.2e-7 either way, and 4%)
+                    f32x4 D[NT], E[NT];
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) D[t] = mfma(lo, B[t][j], zero);
+                    for (int t = 0; t < NT; ++t) D[t] = mfma(hi, B[t][j], zero);
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) D[t] = mfma(mid, B[t][j], D[t]);
+                    for (int t = 0; t < NT; ++t) E[t] = mfma(mid, B[t][j], zero);
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) D[t] = mfma(hi, B[t][j], D[t]);
+                    for (int t = 0; t < NT; ++t) E[t] = mfma(lo, B[t][j], E[t]);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) D[t] += E[t];
                     scaled(D, j);
                 }
             }

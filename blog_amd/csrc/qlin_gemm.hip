@@ -307,7 +307,7 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
         f32x4 dx;
     };
     struct Operands {
-        u32x4 part[Q81 ? 1 : 3];  // smallest first
+        u32x4 part[Q81 ? 1 : 3];  // largest first
         f32x4 dx;
     };
     auto load_raw = [&](const uint4 *buf, int c, int i) {
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(kThreads, G::waves) void gemm_kernel(const GemmArgs
             o.part[0] = r.v[0];
             o.dx = r.dx;
         } else {
-            split3(__builtin_bit_cast(f32x4, r.v[0]), __builtin_bit_cast(f32x4, r.v[1]), o.part[2], o.part[1], o.part[0]);
+            split3(__builtin_bit_cast(f32x4, r.v[0]), __builtin_bit_cast(f32x4, r.v[1]), o.part[0], o.part[1], o.part[2]);
         }
         return o;
     };

@@ -720,6 +720,22 @@ def test_rows_of_f32_over_the_whole_range(qtype, N, m):
     assert (got[6][w0 != 0] == -np.sign(w0[w0 != 0]) * np.inf).all()
 
 
+@pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 896, 4096, 100), (Q6_K, 896, 4096, 100), (Q4_0, 1024, 2048, 60),
+                                         (Q8_0, 8300, 2048, 130), (Q5_0, 14400, 2048, 260)])
+def test_rows_of_f32_mean_error(qtype, N, K, m):
+    """Rounding has no direction: over all outputs the errors average out.  Their spread is about 1e-7 of the mean
+    magnitude, that of the mean over 6e4 outputs and more 4e-10; parts that an MFMA cuts off towards minus infinity
+    are allowed below 2^-8 of the rounding to f32 (2e-8), not at it (3e-8 to 8e-8)."""
+    w, rb, vals = qgen.random_matrix(qtype, N, K, seed=595)
+    x = qgen.random_x(m, K, seed=596)
+    banner(f"rows mean error type={qtype} {m}x{K}x{N}")
+    yd = empty_f32(m, N)
+    qlin.quant_matmul(qtype, dev(w), rb, dev(x), yd, N, K, m)
+    ref = (torch.from_numpy(x).cuda().double() @ torch.from_numpy(vals).cuda().double().t().contiguous())
+    mean = ((yd.double() - ref).mean() / ref.abs().mean()).item()
+    assert abs(mean) <= 2e-8, mean
+
+
 @pytest.mark.parametrize("qtype,N,K,m", [(Q8_0, 100, 256, 9), (Q5_0, 100, 256, 9), (Q4_0, 100, 256, 9),
                                          (Q6_K, 100, 512, 9), (Q8_0, 8300, 224, 130), (Q4_0, 14400, 1056, 300)])
 def test_rows_of_f32_infinite_block_scale(qtype, N, K, m):
