@@ -27,8 +27,9 @@
 // 618 -> 149 us against the f32 matrix cores with the weights decoded per 16 tokens (an fp16 pair of x under a
 // scale per token: 155 and 132 us, but not exact); Q8_1 activations, Q8_0 [14336, 4096] at 512 tokens 303 -> 121 us
 // against the 64-token tiles (155 with d8 q as an fp16 pair).  What bounds it: the step's chain (barrier, reads,
-// splits, products, staging writes); per step and SIMD the large tiles' vector instructions take about 3400
-// cycles, the matrix ones 3100, of 6500.
+// splits, products, staging writes).  At [14336, 4096] x 512 vector instructions take 77% of an active SIMD's cycles
+// and the matrix cores 54% (SQ_INSTS_VALU, SQ_VALU_MFMA_BUSY_CYCLES); 50 fewer of 450 vector instructions a step (Q4_0
+// nibbles by v_cvt_off_f32_i4) and the splits spread between the MFMAs both left the times as they were.
 //
 // Blocks and rows are only 2-byte aligned in general; weights are read as wide loads at that alignment.
 #include "qlin_bf16x3.hpp"
